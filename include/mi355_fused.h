@@ -190,6 +190,23 @@ int mi355_w8a16_linear_fwd(const void* x, const void* w_q, const void* scale, co
                            void* stream);
 
 /*
+ * The same with a workspace, which lets calls of 17 to about 1500 rows whose
+ * output is narrow split K over the GPU (two kernels, no allocation).
+ * mi355_w8a16_linear_workspace returns the bytes such a call wants on the
+ * current device, 0 where it would not use them; `workspace` is 16-byte
+ * aligned device memory of `workspace_bytes` that no other work touches until
+ * the call's kernels end (its contents need no preparation and are left
+ * undefined).  NULL, or fewer bytes than wanted, runs mi355_w8a16_linear_fwd.
+ */
+int64_t mi355_w8a16_linear_workspace(int64_t rows, int64_t k, int64_t n);
+int mi355_w8a16_linear_ws_fwd(const void* x, const void* w_q, const void* scale, const void* bias, void* out,
+                              int64_t rows, int64_t k, int64_t n,
+                              int64_t x_row_stride, int64_t w_row_stride, int64_t out_row_stride,
+                              int x_dtype, int scale_dtype, int bias_dtype, int out_dtype,
+                              void* workspace, int64_t workspace_bytes,
+                              void* stream);
+
+/*
  * Int8 gate/up projections fused with SiLU-and-mul (W8A16 weights), per row
  * m and output feature n:
  *   g[m,n] = (sum_k x[m,k] * wq_gate[n,k]) * scale_gate[n]     (fp32 sums)
@@ -270,6 +287,15 @@ int mi355_linear16_fwd(const void* x, const void* weight, const void* bias, void
                        int64_t x_row_stride, int64_t w_row_stride, int64_t out_row_stride,
                        int dtype, int bias_dtype, int out_dtype,
                        void* stream);
+
+/* The same with a workspace: the rules of mi355_w8a16_linear_ws_fwd. */
+int64_t mi355_linear16_workspace(int64_t rows, int64_t k, int64_t n);
+int mi355_linear16_ws_fwd(const void* x, const void* weight, const void* bias, void* out,
+                          int64_t rows, int64_t k, int64_t n,
+                          int64_t x_row_stride, int64_t w_row_stride, int64_t out_row_stride,
+                          int dtype, int bias_dtype, int out_dtype,
+                          void* workspace, int64_t workspace_bytes,
+                          void* stream);
 
 #ifdef __cplusplus
 }

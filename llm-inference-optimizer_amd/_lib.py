@@ -26,7 +26,9 @@ DTYPE_CODE = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
 
 EXPORTED_SYMBOLS = ("mi355_abi_version", "mi355_last_error", "mi355_rmsnorm_fwd", "mi355_add_rmsnorm_fwd",
                     "mi355_silu_mul_fwd", "mi355_gate_up_silu_fwd", "mi355_w8a16_linear_fwd",
-                    "mi355_quantize_int8_fwd", "mi355_gate_up_silu_w8a16_fwd", "mi355_linear16_fwd")
+                    "mi355_quantize_int8_fwd", "mi355_gate_up_silu_w8a16_fwd", "mi355_linear16_fwd",
+                    "mi355_w8a16_linear_workspace", "mi355_w8a16_linear_ws_fwd", "mi355_linear16_workspace",
+                    "mi355_linear16_ws_fwd")
 
 
 class KernelLibraryMissing(RuntimeError):
@@ -73,6 +75,13 @@ def _declare(L: ctypes.CDLL, path: Path) -> ctypes.CDLL:
     L.mi355_gate_up_silu_w8a16_fwd.restype = i32
     L.mi355_linear16_fwd.argtypes = [vp, vp, vp, vp, i64, i64, i64, i64, i64, i64, i32, i32, i32, vp]
     L.mi355_linear16_fwd.restype = i32
+    for name in ("mi355_w8a16_linear_workspace", "mi355_linear16_workspace"):
+        f = getattr(L, name)
+        f.argtypes, f.restype = [i64, i64, i64], i64
+    L.mi355_w8a16_linear_ws_fwd.argtypes = [*L.mi355_w8a16_linear_fwd.argtypes[:-1], vp, i64, vp]
+    L.mi355_w8a16_linear_ws_fwd.restype = i32
+    L.mi355_linear16_ws_fwd.argtypes = [*L.mi355_linear16_fwd.argtypes[:-1], vp, i64, vp]
+    L.mi355_linear16_ws_fwd.restype = i32
     ver = L.mi355_abi_version()
     if ver != ABI_VERSION:
         raise KernelLibraryMissing(f"{path} has ABI version {ver}, expected {ABI_VERSION}; rebuild it")

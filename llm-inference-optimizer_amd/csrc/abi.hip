@@ -25,11 +25,14 @@ int gate_up_silu_launch(const void* x, const void* wg, const void* wu, void* out
 
 int w8a16_launch(const void* x, const void* q, const void* scale, const void* bias, void* out, int rows, int k,
                  int n, int64_t xs, int64_t qs, int64_t os, int x_dtype, int scale_dtype, int bias_dtype,
-                 int out_dtype, hipStream_t stream);
+                 int out_dtype, void* work, int64_t work_bytes, hipStream_t stream);
 int quantize_int8_launch(const void* w, void* q, void* scale, int64_t n, int k, int64_t ws, int64_t qs, int w_dtype,
                          hipStream_t stream);
 int linear16_launch(const void* x, const void* w, const void* bias, void* out, int rows, int k, int n, int64_t xs,
-                    int64_t ws, int64_t os, int dtype, int bias_dtype, int out_dtype, hipStream_t stream);
+                    int64_t ws, int64_t os, int dtype, int bias_dtype, int out_dtype, void* work, int64_t work_bytes,
+                    hipStream_t stream);
+// fp32 scratch bytes the split-K kernels want (0: none), for weight_bytes per weight
+int64_t split_workspace(int64_t rows, int64_t k, int64_t n, int weight_bytes);
 int gate_up_silu_w8a16_launch(const void* x, const void* qg, const void* qu, const void* sg, const void* su, void* out,
                               int rows, int k, int n, int64_t xs, int64_t qs, int64_t os, int x_dtype,
                               int scale_dtype, int out_dtype, hipStream_t stream);
@@ -241,10 +244,15 @@ MI355_EXPORT int mi355_gate_up_silu_fwd(const void* x, const void* w_gate, const
                                     out_dtype, static_cast<hipStream_t>(stream));
 }
 
-MI355_EXPORT int mi355_w8a16_linear_fwd(const void* x, const void* w_q, const void* scale, const void* bias,
-                                        void* out, int64_t rows, int64_t k, int64_t n, int64_t x_row_stride,
-                                        int64_t w_row_stride, int64_t out_row_stride, int x_dtype, int scale_dtype,
-                                        int bias_dtype, int out_dtype, void* stream) {
+MI355_EXPORT int64_t mi355_w8a16_linear_workspace(int64_t rows, int64_t k, int64_t n) {
+  return mi355::split_workspace(rows, k, n, 1);
+}
+
+MI355_EXPORT int mi355_w8a16_linear_ws_fwd(const void* x, const void* w_q, const void* scale, const void* bias,
+                                           void* out, int64_t rows, int64_t k, int64_t n, int64_t x_row_stride,
+                                           int64_t w_row_stride, int64_t out_row_stride, int x_dtype, int scale_dtype,
+                                           int bias_dtype, int out_dtype, void* workspace, int64_t workspace_bytes,
+                                           void* stream) {
   static const char* fn = "mi355_w8a16_linear_fwd";
   mi355::g_error[0] = '\0';
   if (!valid_dtype(x_dtype) || !valid_dtype(scale_dtype) || !valid_dtype(out_dtype) ||
@@ -275,6 +283,10 @@ MI355_EXPORT int mi355_w8a16_linear_fwd(const void* x, const void* w_q, const vo
     set_error("%s: null pointer", fn);
     return MI355_ERR_INVALID;
   }
+  if (workspace != nullptr && (!mi355::aligned16(workspace) || workspace_bytes < 0)) {
+    set_error("%s: the workspace must be 16-byte aligned and its size >= 0", fn);
+    return MI355_ERR_INVALID;
+  }
   // Buffer descriptors span at most 128 rows of x or of w_q (< 2^32 bytes);
   // grids hold ceil(n / 128) x ceil(rows / 64) workgroups or more.
   if (x_row_stride >= (int64_t{1} << 23) || w_row_stride >= (int64_t{1} << 24) || n > 0x7fffffff - 128 ||
@@ -293,7 +305,15 @@ MI355_EXPORT int mi355_w8a16_linear_fwd(const void* x, const void* w_q, const vo
   }
   return mi355::w8a16_launch(x, w_q, scale, bias, out, static_cast<int>(rows), static_cast<int>(k),
                              static_cast<int>(n), x_row_stride, w_row_stride, out_row_stride, x_dtype, scale_dtype,
-                             bias_dtype, out_dtype, static_cast<hipStream_t>(stream));
+                             bias_dtype, out_dtype, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+MI355_EXPORT int mi355_w8a16_linear_fwd(const void* x, const void* w_q, const void* scale, const void* bias,
+                                        void* out, int64_t rows, int64_t k, int64_t n, int64_t x_row_stride,
+                                        int64_t w_row_stride, int64_t out_row_stride, int x_dtype, int scale_dtype,
+                                        int bias_dtype, int out_dtype, void* stream) {
+  return mi355_w8a16_linear_ws_fwd(x, w_q, scale, bias, out, rows, k, n, x_row_stride, w_row_stride, out_row_stride,
+                                   x_dtype, scale_dtype, bias_dtype, out_dtype, nullptr, 0, stream);
 }
 
 MI355_EXPORT int mi355_gate_up_silu_w8a16_fwd(const void* x, const void* wq_gate, const void* wq_up,
@@ -381,9 +401,14 @@ MI355_EXPORT int mi355_quantize_int8_fwd(const void* w, void* w_q, void* scale, 
                                      static_cast<hipStream_t>(stream));
 }
 
-MI355_EXPORT int mi355_linear16_fwd(const void* x, const void* weight, const void* bias, void* out, int64_t rows,
-                                    int64_t k, int64_t n, int64_t x_row_stride, int64_t w_row_stride,
-                                    int64_t out_row_stride, int dtype, int bias_dtype, int out_dtype, void* stream) {
+MI355_EXPORT int64_t mi355_linear16_workspace(int64_t rows, int64_t k, int64_t n) {
+  return mi355::split_workspace(rows, k, n, 2);
+}
+
+MI355_EXPORT int mi355_linear16_ws_fwd(const void* x, const void* weight, const void* bias, void* out, int64_t rows,
+                                       int64_t k, int64_t n, int64_t x_row_stride, int64_t w_row_stride,
+                                       int64_t out_row_stride, int dtype, int bias_dtype, int out_dtype,
+                                       void* workspace, int64_t workspace_bytes, void* stream) {
   static const char* fn = "mi355_linear16_fwd";
   mi355::g_error[0] = '\0';
   if (!valid_dtype(dtype) || !valid_dtype(out_dtype) || (bias != nullptr && !valid_dtype(bias_dtype))) {
@@ -412,6 +437,10 @@ MI355_EXPORT int mi355_linear16_fwd(const void* x, const void* weight, const voi
     set_error("%s: null pointer", fn);
     return MI355_ERR_INVALID;
   }
+  if (workspace != nullptr && (!mi355::aligned16(workspace) || workspace_bytes < 0)) {
+    set_error("%s: the workspace must be 16-byte aligned and its size >= 0", fn);
+    return MI355_ERR_INVALID;
+  }
   // Buffer descriptors span at most 256 rows of x or of the weights (< 2^32
   // bytes); grids hold ceil(n / 8) x ceil(rows / 32) workgroups or more.
   if (x_row_stride >= (int64_t{1} << 22) || w_row_stride >= (int64_t{1} << 22) || n > 0x7fffffff - 256 ||
@@ -429,5 +458,12 @@ MI355_EXPORT int mi355_linear16_fwd(const void* x, const void* weight, const voi
   }
   return mi355::linear16_launch(x, weight, bias, out, static_cast<int>(rows), static_cast<int>(k),
                                 static_cast<int>(n), x_row_stride, w_row_stride, out_row_stride, dtype, bias_dtype,
-                                out_dtype, static_cast<hipStream_t>(stream));
+                                out_dtype, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+MI355_EXPORT int mi355_linear16_fwd(const void* x, const void* weight, const void* bias, void* out, int64_t rows,
+                                    int64_t k, int64_t n, int64_t x_row_stride, int64_t w_row_stride,
+                                    int64_t out_row_stride, int dtype, int bias_dtype, int out_dtype, void* stream) {
+  return mi355_linear16_ws_fwd(x, weight, bias, out, rows, k, n, x_row_stride, w_row_stride, out_row_stride, dtype,
+                               bias_dtype, out_dtype, nullptr, 0, stream);
 }

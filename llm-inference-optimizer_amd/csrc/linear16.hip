@@ -11,19 +11,24 @@
 // bandwidth (about 21 us for the 27.5 MB down projection of Qwen2.5-1.5B at
 // 1 to 8 rows on MI355X).
 //
-// Three kernels, picked by the launcher:
+// Four kernels, picked by the launcher:
 //   w8a16_stream      rows <= 16 (decode; w8a16_stream.h with one 16-bit
-//                     matrix), and 17 - 64 where the small tiled shapes do not
-//                     pay: lane-coalesced weight streaming, every weight byte
-//                     read once per call, MFMA (v_mfma_f32_16x16x32_*).
+//                     matrix), and 17 - 64 where neither the small tiled
+//                     shapes nor split K pay: lane-coalesced weight
+//                     streaming, every weight byte read once per call, MFMA
+//                     (v_mfma_f32_16x16x32_*).
 //   tiled_gemm        more rows, and 17 - 64 on wide outputs: the LDS-tiled
 //                     MFMA GEMM of tiled_gemm.h with the weights as a 16-bit B
 //                     operand and the bias in its epilogue (EPI_LINEAR).
-//   linear16_generic  any k, stride or alignment the two above cannot take:
+//   split_k.h         from 17 rows, given a workspace, where the output holds
+//                     too few tiles for the CUs: the same GEMM over ranges of
+//                     K and a second pass that adds them.
+//   linear16_generic  any k, stride or alignment the others cannot take:
 //                     one wave per (output feature, 4 rows of x), fp32 fma.
 // Under the C ABI's limits (row strides < 2^22 elements) the buffer
-// descriptors of the first two always span their inputs.
+// descriptors of all but the last always span their inputs.
 #include "common.h"
+#include "split_k.h"
 #include "tiled_gemm.h"
 #include "w8a16_stream.h"
 
@@ -93,10 +98,7 @@ bool l16_tiled_fits(const L16Params& p) {
          static_cast<int64_t>((p.rows + 63) / 64) * ((p.n + 63) / 64) < (int64_t{1} << 31);
 }
 
-template <typename T, typename TO, int WGM, int WGN, int FM, int FN, int S, int RING = 0>
-int l16_tiled_cfg(const L16Params& p, hipStream_t s) {
-  using C = tiled::Cfg<T, tiled::B_16, TO, WGM, WGN, FM, FN, tiled::EPI_LINEAR, S>;
-  static_assert(C::LDS <= 160 * 1024, "LDS per workgroup");
+tiled::Params l16_tiled_params(const L16Params& p) {
   tiled::Params tp{};
   tp.x = p.x;
   tp.b0 = p.w;
@@ -111,44 +113,58 @@ int l16_tiled_cfg(const L16Params& p, hipStream_t s) {
   tp.os = p.os;
   tp.sdt = MI355_F32;
   tp.bdt = p.bdt;
+  return tp;
+}
+
+template <typename T, typename TO, int WGM, int WGN, int FM, int FN, int S, int RING = 0, int XR = 1>
+int l16_tiled_cfg(const L16Params& p, hipStream_t s) {
+  using C = tiled::Cfg<T, tiled::B_16, TO, WGM, WGN, FM, FN, tiled::EPI_LINEAR, S>;
+  static_assert(C::LDS <= 160 * 1024, "LDS per workgroup");
+  tiled::Params tp = l16_tiled_params(p);
   tp.tiles_m = (p.rows + C::BM - 1) / C::BM;
   tp.tiles_n = (p.n + C::BN - 1) / C::BN;
   tp.group_m = tp.tiles_m < 4 ? tp.tiles_m : 4;
   void* args[] = {&tp};
   // all LDS is static (no dynamic shared memory)
   return hip_status(hipLaunchKernel(reinterpret_cast<const void*>(tiled::tiled_gemm<T, tiled::B_16, TO, WGM, WGN, FM, FN,
-                                                                                      tiled::EPI_LINEAR, S, RING>),
+                                                                                      tiled::EPI_LINEAR, S, RING, 0, XR>),
                                     dim3(static_cast<unsigned>(tp.tiles_m * tp.tiles_n)), dim3(C::BLOCK), args, 0, s),
                     "linear16 tiled launch");
 }
 
-// Tiled shapes (16-bit B, one matrix): 64 x 64 tiles on small grids, 128 x
-// 128 (8 waves, 3 stages) otherwise.
+// Unsplit tiles of more than 64 rows, by split_plan's predicted times: 64 x
+// 64 (4 waves, 4 stages), then on the sub-step ring 64 x 128 (4 stages), 128
+// x 128 (3), 256 x 128 and 256 x 256 (2).  (The rule before -- 64 x 64 below
+// 128 tiles of 128 x 128, else those in the step pipeline -- took 1.5B q/o
+// 1000 rows 12.6 us, now 11.2; 3B 16.9, now 12.9; the 14B q/o 333 rows 45.1,
+// now 36.8.)
 template <typename T, typename TO>
-int l16_tiled(const L16Params& p, hipStream_t s) {
-  const int64_t t128 = static_cast<int64_t>((p.rows + 127) / 128) * ((p.n + 127) / 128);
-  if (t128 < 128) return l16_tiled_cfg<T, TO, 2, 2, 1, 1, 4>(p, s);
-  return l16_tiled_cfg<T, TO, 2, 4, 2, 1, 3>(p, s);
+int l16_tiled(const L16Params& p, int shape, hipStream_t s) {
+  switch (shape) {
+    case 0: return l16_tiled_cfg<T, TO, 2, 2, 1, 1, 4>(p, s);
+    case 1: return l16_tiled_cfg<T, TO, 2, 4, 1, 1, 4, 1>(p, s);
+    case 2: return l16_tiled_cfg<T, TO, 2, 4, 2, 1, 3, 1>(p, s);
+    case 3: return l16_tiled_cfg<T, TO, 2, 4, 4, 1, 2, 1>(p, s);
+    default: return l16_tiled_cfg<T, TO, 2, 4, 4, 2, 2, 1>(p, s);
+  }
 }
 
 // Small tiled shapes: 32 x 64 (2 waves) or, for n > 10000, 32 x 128 (4 waves)
 // up to 32 rows; 64 x 64 (4 waves) up to 64; 4 stages.  From a sweep over
-// the Qwen2.5-1.5B / 7B down and o projections at 16 - 64 rows: at 17 - 32
-// rows they lose to split-K weight streaming on these narrow outputs (1.5B
-// down, 32 rows: 38.0 vs 22.3 us) unless the output has >= 128 tile
-// columns; at 33 - 64 rows, where streaming re-reads the weights per 32-row
-// tile, they win (7B down, 48 rows: 85.5 vs 101.6 us; 7B o 19.4 vs 22.6).
+// the Qwen2.5-1.5B / 7B down and o projections at 16 - 64 rows: on narrow
+// outputs (fewer than 128 tile columns) they lose to split-K weight
+// streaming (1.5B down, 32 rows: 38.0 vs 22.3 us).
 template <typename T, typename TO>
 int l16_tiled_small(const L16Params& p, hipStream_t s) {
   if (p.rows <= 32) {
-    if (p.n > 10000) return l16_tiled_cfg<T, TO, 1, 4, 1, 1, 4>(p, s);
-    return l16_tiled_cfg<T, TO, 1, 2, 1, 1, 4>(p, s);
+    if (p.n > 10000) return l16_tiled_cfg<T, TO, 1, 4, 1, 1, 4, 0, 0>(p, s);
+    return l16_tiled_cfg<T, TO, 1, 2, 1, 1, 4, 0, 0>(p, s);
   }
-  return l16_tiled_cfg<T, TO, 2, 2, 1, 1, 4>(p, s);
+  return l16_tiled_cfg<T, TO, 2, 2, 1, 1, 4, 0, 0>(p, s);
 }
 
 template <typename T, typename TO>
-int l16_typed(const L16Params& p, hipStream_t s, int cus) {
+int l16_typed(const L16Params& p, void* work, int64_t work_bytes, hipStream_t s, int cus) {
   const bool vec = p.k % 8 == 0 && p.ws % 8 == 0 && p.xs % 8 == 0 && aligned16(p.x) && aligned16(p.w);
   if (!vec) {
     const int64_t waves = static_cast<int64_t>(p.n) * ((p.rows + kGenRows - 1) / kGenRows);
@@ -170,33 +186,40 @@ int l16_typed(const L16Params& p, hipStream_t s, int cus) {
   }
   const W8Params w{p.x, p.w, nullptr, p.bias, p.out, p.rows, p.k, p.n, p.xs, p.ws, p.os, MI355_F32, p.bdt,
                    nullptr, nullptr};
+  const tiled::SplitPlan sp = tiled::split_plan(p.rows, p.k, p.n, 2, cus);
+  if (sp.tile >= 0 && work != nullptr && work_bytes >= tiled::split_bytes(sp, p.rows, p.n))
+    return tiled::split_k_launch<T, tiled::B_16, TO, tiled::EPI_LINEAR>(l16_tiled_params(p), sp,
+                                                                         static_cast<float*>(work), s);
   if (p.rows <= 64) {
     const int bn = (p.rows <= 32 && p.n > 10000) ? 128 : 64;
     if (p.rows <= 16 || (p.n + bn - 1) / bn < 128)
       return w8_stream_launch<T, TO, false, 2>(w, l16_stream_plan(p.rows, p.k, p.n, cus), s);
     return l16_tiled_small<T, TO>(p, s);
   }
-  // More rows: the tiled GEMM.  (32-row skinny tiles with split K re-read
-  // 16-bit weights per tile: at 96 - 256 rows of the Qwen2.5-1.5B / 7B down
-  // and o projections they measured 1.7 - 4.0x slower than the tiled GEMM
-  // even on small grids, e.g. 7B down, 256 rows 350.9 vs 87.8 us.)
-  return l16_tiled<T, TO>(p, s);
+  return l16_tiled<T, TO>(p, sp.direct, s);
 }
 
 }  // namespace
 
 int linear16_launch(const void* x, const void* w, const void* bias, void* out, int rows, int k, int n, int64_t xs,
-                    int64_t ws, int64_t os, int dtype, int bias_dtype, int out_dtype, hipStream_t stream) {
+                    int64_t ws, int64_t os, int dtype, int bias_dtype, int out_dtype, void* work, int64_t work_bytes,
+                    hipStream_t stream) {
   int cus = 0;
   const int st = compute_units(&cus);
   if (st != MI355_OK) return st;
   const L16Params p{x, w, bias, out, rows, k, n, xs, ws, os, bias ? bias_dtype : -1};
-  if (dtype == MI355_F16 && out_dtype == MI355_F16) return l16_typed<F16, F16>(p, stream, cus);
-  if (dtype == MI355_F16 && out_dtype == MI355_F32) return l16_typed<F16, F32>(p, stream, cus);
-  if (dtype == MI355_BF16 && out_dtype == MI355_BF16) return l16_typed<BF16, BF16>(p, stream, cus);
-  if (dtype == MI355_BF16 && out_dtype == MI355_F32) return l16_typed<BF16, F32>(p, stream, cus);
+  if (dtype == MI355_F16 && out_dtype == MI355_F16) return l16_typed<F16, F16>(p, work, work_bytes, stream, cus);
+  if (dtype == MI355_F16 && out_dtype == MI355_F32) return l16_typed<F16, F32>(p, work, work_bytes, stream, cus);
+  if (dtype == MI355_BF16 && out_dtype == MI355_BF16) return l16_typed<BF16, BF16>(p, work, work_bytes, stream, cus);
+  if (dtype == MI355_BF16 && out_dtype == MI355_F32) return l16_typed<BF16, F32>(p, work, work_bytes, stream, cus);
   set_error("mi355_linear16_fwd: unsupported dtype pair (in=%d, out=%d)", dtype, out_dtype);
   return MI355_ERR_UNSUPPORTED;
+}
+
+int64_t split_workspace(int64_t rows, int64_t k, int64_t n, int weight_bytes) {
+  int cus = 0;
+  if (rows <= 16 || k < 1 || n < 1 || compute_units(&cus) != MI355_OK) return 0;
+  return tiled::split_bytes(tiled::split_plan(rows, k, n, weight_bytes, cus), rows, n);
 }
 
 }  // namespace mi355

@@ -7,6 +7,7 @@
 #include <cstdarg>
 #include <cstdio>
 
+#include "../split_k.h"
 #include "../w8a16_stream.h"
 
 namespace mi355 {
@@ -251,4 +252,18 @@ extern "C" __attribute__((visibility("default"))) void mi355_probe_gate_up16_str
   out4[1] = sp.r4;
   out4[2] = sp.waves;
   out4[3] = sp.u;
+}
+
+// The split-K plan (split_plan) of a [rows, k] x [n, k] product with wb-byte
+// weights on `cus` CUs: out4 = {tile (< 0: not split), K ranges, the tile's
+// rows, its columns}; returns the workspace bytes.
+extern "C" __attribute__((visibility("default"))) long long mi355_probe_split_plan(long long rows, long long k,
+                                                                                    long long n, int wb, int cus,
+                                                                                    int* out4) {
+  const mi355::tiled::SplitPlan sp = mi355::tiled::split_plan(rows, k, n, wb, cus);
+  out4[0] = sp.tile;
+  out4[1] = sp.splits;
+  out4[2] = sp.tile < 0 ? 0 : mi355::tiled::kSplitCost16[sp.tile].bm;
+  out4[3] = sp.tile < 0 ? 0 : mi355::tiled::kSplitCost16[sp.tile].bn;
+  return mi355::tiled::split_bytes(sp, rows, n);
 }

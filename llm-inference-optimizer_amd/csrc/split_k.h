@@ -1,0 +1,220 @@
+// Split-K GEMM for gfx950: the LDS-tiled kernel of tiled_gemm.h over S ranges
+// of K (EPI_PART, fp32 sums to a workspace), then one pass that adds the S
+// sums of each output in range order and applies the caller's epilogue; plus
+// the plan that picks tile and S, for the W8A16 linear (w8a16.hip) and the
+// 16-bit linear (linear16.hip).
+//
+// Why.  Up to a few hundred rows the output of a down projection (n 896 -
+// 5120) holds 12 - 100 tiles, and the weights (k 4864 - 18944) are a deep
+// stream each tile reads alone: 256 CUs sit mostly idle behind a serial chain
+// of 76 - 296 K steps.  S = CUs / tiles ranges give every CU a workgroup and
+// cut the chain by S, for 8 S rows n bytes of extra traffic (fp32 sums
+// written once and read once, L2 and Infinity Cache hits) and a second
+// launch.  Measured on MI355X, weights from HBM, before (the stream kernel up
+// to 64 rows, unsplit tiles beyond) and after, both passes:
+//   7B down (18944 -> 3584), 16-bit:  64 rows 80.6 -> 32.0 us, 200 rows 79.3
+//     -> 52.3, 512 rows 153 -> 85.4, 1000 rows 168 -> 134 (1.01 PFLOP/s);
+//     int8: 64 rows 82.3 -> 25.8, 200 rows 82.2 -> 46.3, 512 rows 123 -> 88
+//   1.5B down (8960 -> 1536), 16-bit: 64 rows 19.9 -> 13.3, 200 rows 38.1 ->
+//     18.8, 1000 rows 70.8 -> 46.8; int8: 64 rows 29.1 -> 12.4, 200 rows 38.9
+//     -> 18.3, 1000 rows 49.2 -> 41.9
+// What bounds it: HBM on the weights up to about 64 rows (16-bit: 4.8 TB/s
+// in the first pass alone), per-step latency of one workgroup per CU above;
+// the second pass costs about 3 us and its launch about 3 more in a stream.
+//
+// Every output's sum is taken in one fixed order (range by range, each in
+// tiled_gemm's order), so equal calls give equal bits.
+#pragma once
+
+#include "common.h"
+#include "tiled_gemm.h"
+
+namespace mi355 {
+namespace tiled {
+
+// EPI: the caller's unsplit epilogue (EPI_W8 or EPI_LINEAR); VEC: columns per
+// thread (4 with 16-byte loads, or 1).  Bound by latency: a thread's loads of
+// 4 ranges are in flight together.
+template <typename TO, int EPI, int VEC>
+__global__ __launch_bounds__(256) void split_k_reduce(const Params p) {
+  static_assert(EPI == EPI_W8 || EPI == EPI_LINEAR, "one matrix");
+  const int nv = p.n / VEC;
+  const int64_t id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (id >= static_cast<int64_t>(nv) * p.rows) return;
+  const int64_t m = id / nv;
+  const int n = static_cast<int>(id - m * nv) * VEC;
+  const int64_t plane = static_cast<int64_t>(p.rows) * p.n;
+  const float* src = p.part + m * p.n + n;
+  float acc[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) acc[e] = 0.f;
+#pragma unroll 4
+  for (int s = 0; s < p.splits; ++s) {
+    if constexpr (VEC == 4) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(src + s * plane);
+      acc[0] += v.x; acc[1] += v.y; acc[2] += v.z; acc[3] += v.w;
+    } else {
+      acc[0] += src[s * plane];
+    }
+  }
+  float v[VEC];
+#pragma unroll
+  for (int e = 0; e < VEC; ++e) {
+    if constexpr (EPI == EPI_W8) {
+      const float sc = load_dyn(p.scale, n + e, p.sdt);
+      v[e] = p.bdt >= 0 ? __builtin_fmaf(acc[e], sc, load_dyn(p.bias, n + e, p.bdt)) : acc[e] * sc;
+    } else {
+      v[e] = p.bdt >= 0 ? acc[e] + load_dyn(p.bias, n + e, p.bdt) : acc[e];
+    }
+  }
+  const int64_t o = m * p.os + n;
+  if constexpr (VEC == 4) {
+    if constexpr (is_half_width<TO>::value) {
+      const f32x2 lo = {v[0], v[1]}, hi = {v[2], v[3]};
+      *reinterpret_cast<u32x2*>(static_cast<typename TO::bits*>(p.out) + o) = u32x2{narrow2<TO>(lo), narrow2<TO>(hi)};
+    } else {
+      *reinterpret_cast<u32x4*>(static_cast<float*>(p.out) + o) =
+          u32x4{as_u32(v[0]), as_u32(v[1]), as_u32(v[2]), as_u32(v[3])};
+    }
+  } else {
+    store_elem<TO>(p.out, o, v[0]);
+  }
+}
+
+// ---------------------------------------------------------------- the plan
+
+// Time of one call in us over a tile shape: c0 + step * (K steps a CU runs
+// one after another) + part * (MB of fp32 sums written and read) + weight *
+// (MB of weights).  Least-squares fits of a sweep on MI355X over the
+// Qwen2.5-0.5B to 14B down projections and square projections (896 - 5120
+// outputs, k 1536 - 18944) at 24 - 1500 rows, weights rotated through HBM:
+// mean error 2 - 5% per split tile, 5 - 12% per unsplit one; the plan's pick
+// is within 1.05x of the best measured shape on geometric average above 64
+// rows.
+struct TileCost {
+  int bm, bn;
+  double c0, step, part, weight;
+};
+enum { SPLIT_TILES = 5, DIRECT_TILES = 5 };
+// Split tiles: 32 x 128, 64 x 64, 64 x 128, 128 x 128, 256 x 256.
+constexpr TileCost kSplitCost16[SPLIT_TILES] = {
+    {32, 128, 5.4, 0.256, 0.199, 0.113}, {64, 64, 5.0, 0.202, 0.288, 0.091},  {64, 128, 5.3, 0.310, 0.307, 0.087},
+    {128, 128, 6.8, 0.440, 0.230, 0.060}, {256, 256, 2.8, 1.406, 0.219, 0.054}};
+constexpr TileCost kSplitCost8[SPLIT_TILES] = {
+    {32, 128, 6.4, 0.235, 0.249, 0.082}, {64, 64, 6.3, 0.226, 0.281, 0.053},  {64, 128, 6.8, 0.284, 0.320, 0.054},
+    {128, 128, 8.9, 0.430, 0.226, 0.011}, {256, 256, 4.1, 1.659, 0.211, 0.005}};
+// Unsplit tiles: 64 x 64, 64 x 128, 128 x 128, 256 x 128, 256 x 256.
+constexpr TileCost kDirectCost16[DIRECT_TILES] = {{64, 64, 2.9, 0.206, 0, 0.155},
+                                                  {64, 128, 0.7, 0.300, 0, 0.242},
+                                                  {128, 128, 1.4, 0.389, 0, 0.255},
+                                                  {256, 128, 0, 0.791, 0, 0.408},
+                                                  {256, 256, 5.2, 1.149, 0, 0.277}};
+constexpr TileCost kDirectCost8[DIRECT_TILES] = {{64, 64, 6.5, 0.176, 0, 0.258},
+                                                 {64, 128, 5.6, 0.258, 0, 0.190},
+                                                 {128, 128, 6.3, 0.344, 0, 0.194},
+                                                 {256, 128, 5.3, 0.650, 0, 0.431},
+                                                 {256, 256, 11.8, 1.162, 0, 0.188}};
+// The weight-streaming kernel at 17 - 24, 25 - 32, 33 - 48 and 49 - 64 rows
+// (from 49 rows of more than 8 MB of int8 weights: the kernels that run
+// there): fixed us, us per MB of weights.
+constexpr double kStreamCost16[4][2] = {{3.1, 0.24}, {3.4, 0.29}, {4.1, 0.44}, {4.9, 0.52}};
+constexpr double kStreamCost8[4][2] = {{3.5, 0.36}, {4.1, 0.44}, {4.5, 0.69}, {4.9, 0.90}};
+
+struct SplitPlan {
+  int tile;     // index into the split table; < 0: the unsplit kernels are faster
+  int splits;   // K ranges, >= 2
+  double cost;  // predicted us
+  int direct;   // the fastest unsplit tile (index into the direct table)
+};
+
+// The fastest split tile and count for [rows, k] x [n, k] (wb: bytes per
+// weight), against the fastest unsplit kernel at that size.  One workgroup
+// per CU: S = CUs / tiles, no more than 32, at least 4 K steps each, every
+// range with work.  Splitting has to win by 5% in the prediction; above 64
+// rows from k = 4096 on, where the fits of the unsplit tiles run low, it may
+// lose by 5% (int8 1.5B down, 1000 rows: predicted 44.7 against 44.3 us,
+// measured 41.9 against 49.2).
+inline SplitPlan split_plan(int64_t rows, int64_t k, int64_t n, int wb, int cus) {
+  const auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  const TileCost* sc = wb == 1 ? kSplitCost8 : kSplitCost16;
+  const TileCost* dc = wb == 1 ? kDirectCost8 : kDirectCost16;
+  const double wmb = static_cast<double>(n) * static_cast<double>(k) * wb * 1e-6;
+  const int64_t steps = cdiv(k, 64);
+  SplitPlan best{-1, 1, 1e30, 0};
+  if (rows <= 16) return best;
+  double direct = 1e30;
+  for (int t = 0; t < DIRECT_TILES; ++t) {
+    const int64_t rounds = cdiv(cdiv(rows, dc[t].bm) * cdiv(n, dc[t].bn), cus);
+    const double c = dc[t].c0 + dc[t].step * static_cast<double>(steps * rounds) + dc[t].weight * wmb;
+    if (c < direct) direct = c, best.direct = t;
+  }
+  if (rows <= 64) {
+    const int cls = rows <= 24 ? 0 : (rows <= 32 ? 1 : (rows <= 48 ? 2 : 3));
+    const double* st = wb == 1 ? kStreamCost8[cls] : kStreamCost16[cls];
+    const double c = st[0] + st[1] * wmb;
+    if (c < direct) direct = c;
+  }
+  const double limit = direct * (rows > 64 && k >= 4096 ? 1.05 : 0.95);
+  for (int t = 0; t < SPLIT_TILES; ++t) {
+    const int64_t tiles = cdiv(rows, sc[t].bm) * cdiv(n, sc[t].bn);
+    int64_t s = cus / tiles;
+    if (s > 32) s = 32;
+    if (s > steps / 4) s = steps / 4;
+    if (s < 2) continue;
+    const int64_t per = cdiv(steps, s);
+    s = cdiv(steps, per);
+    if (s < 2) continue;
+    const double pmb = 8e-6 * static_cast<double>(s) * static_cast<double>(rows) * static_cast<double>(n);
+    const double c = sc[t].c0 + sc[t].step * static_cast<double>(per) + sc[t].part * pmb + sc[t].weight * wmb;
+    if (c < best.cost && c < limit) best = SplitPlan{t, static_cast<int>(s), c, best.direct};
+  }
+  return best;
+}
+
+inline int64_t split_bytes(const SplitPlan& sp, int64_t rows, int64_t n) {
+  return sp.tile < 0 ? 0 : static_cast<int64_t>(sizeof(float)) * sp.splits * rows * n;
+}
+
+// ------------------------------------------------------------- the launches
+
+template <typename T, int BK, int WGM, int WGN, int FM, int FN, int S>
+int split_gemm_cfg(const Params& p0, hipStream_t s) {
+  using C = Cfg<T, BK, F32, WGM, WGN, FM, FN, EPI_PART, S>;
+  static_assert(C::LDS <= 160 * 1024, "LDS per workgroup");
+  Params p = p0;
+  p.tiles_m = (p.rows + C::BM - 1) / C::BM;
+  p.tiles_n = (p.n + C::BN - 1) / C::BN;
+  p.group_m = p.tiles_m < 4 ? p.tiles_m : 4;
+  void* args[] = {&p};
+  return hip_status(
+      hipLaunchKernel(reinterpret_cast<const void*>(tiled_gemm<T, BK, F32, WGM, WGN, FM, FN, EPI_PART, S, 1, 0, 1>),
+                      dim3(static_cast<unsigned>(p.tiles_m * p.tiles_n * p.splits)), dim3(C::BLOCK), args, 0, s),
+      "split-K launch");
+}
+
+// Both passes of plan sp; p holds the caller's operands and epilogue.
+template <typename T, int BK, typename TO, int EPI>
+int split_k_launch(Params p, const SplitPlan& sp, float* part, hipStream_t s) {
+  p.part = part;
+  p.splits = sp.splits;
+  int st = MI355_ERR_UNSUPPORTED;
+  switch (sp.tile) {
+    case 0: st = split_gemm_cfg<T, BK, 1, 4, 1, 1, 4>(p, s); break;
+    case 1: st = split_gemm_cfg<T, BK, 2, 2, 1, 1, 4>(p, s); break;
+    case 2: st = split_gemm_cfg<T, BK, 1, 4, 2, 1, 4>(p, s); break;
+    case 3: st = split_gemm_cfg<T, BK, 2, 4, 2, 1, 3>(p, s); break;
+    case 4: st = split_gemm_cfg<T, BK, 2, 4, 4, 2, 2>(p, s); break;
+    default: set_error("split-K: no tile %d", sp.tile);
+  }
+  if (st != MI355_OK) return st;
+  const bool vec = p.n % 4 == 0 && p.os % 4 == 0 && aligned16(p.out);
+  const int64_t threads = static_cast<int64_t>(p.rows) * p.n / (vec ? 4 : 1);
+  void* args[] = {&p};
+  const void* kern = vec ? reinterpret_cast<const void*>(split_k_reduce<TO, EPI, 4>)
+                         : reinterpret_cast<const void*>(split_k_reduce<TO, EPI, 1>);
+  return hip_status(hipLaunchKernel(kern, dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), args, 0, s),
+                    "split-K reduction launch");
+}
+
+}  // namespace tiled
+}  // namespace mi355

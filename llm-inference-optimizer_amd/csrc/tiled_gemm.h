@@ -7,6 +7,7 @@
 //   EPI_LINEAR   out[m, n] = round(acc + bias[n])             b of x's 16-bit type
 //   EPI_SILU  out[m, n] = round(silu(acc_gate) * acc_up)      two 16-bit b
 //   EPI_SILU_W8  out[m, n] = round(silu(acc_gate * scale[n]) * (acc_up * scale1[n]))   two int8 b
+//   EPI_PART  part[s, m, n] = the fp32 sum over K range s     one b (split K; split_k.h adds the ranges)
 //
 // x is [rows, xs] fp16/bf16 and every b is nn.Linear's [n, bs] layout (int8 or
 // x's 16-bit type), used in place.  Arithmetic: 16-bit products, fp32
@@ -83,7 +84,7 @@ namespace tiled {
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
-enum { EPI_W8 = 0, EPI_SILU = 1, EPI_SILU_W8 = 2, EPI_LINEAR = 3 };
+enum { EPI_W8 = 0, EPI_SILU = 1, EPI_SILU_W8 = 2, EPI_LINEAR = 3, EPI_PART = 4 };
 
 enum { B_16 = 0, B_I8 = 1 };
 
@@ -125,6 +126,8 @@ struct Params {
   int sdt, bdt;        // dtype codes of scale and bias (bdt < 0: no bias)
   int tiles_m, tiles_n;
   int group_m;  // m-blocks per group of the tile order (tiles_m: m fastest over the whole range)
+  float* part;  // EPI_PART: [splits][rows][n] fp32 sums
+  int splits;   // EPI_PART: K ranges of ceil(steps / splits) 64-column steps each
 };
 
 template <typename T, int BK, typename TO, int WGM, int WGN, int FM, int FN, int EPI, int S>
@@ -135,7 +138,7 @@ struct Cfg {
   static constexpr int NW = WGM * WGN, NT = 64 * NW;
   static constexpr int BLOCK = NT;  // threads per workgroup
   static constexpr int BM = 32 * FM * WGM, BN = 32 * FN * WGN;
-  static constexpr int NB = (EPI == EPI_W8 || EPI == EPI_LINEAR) ? 1 : 2;  // B matrices
+  static constexpr int NB = (EPI == EPI_W8 || EPI == EPI_LINEAR || EPI == EPI_PART) ? 1 : 2;  // B matrices
   static constexpr int A_BYTES = BM * 128;             // 64 columns of 16-bit x per row
   static constexpr int B_ROW = I8 ? 64 : 128;          // bytes per B row per step in LDS
   static constexpr int B_BYTES = BN * B_ROW;
@@ -232,14 +235,28 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
   const int wm = wave / WGN, wn = wave % WGN;
 
   // Tile of this workgroup: contiguous ranges per XCD, m fastest.
+  constexpr bool PART = EPI == EPI_PART;
   const int ntiles = p.tiles_m * p.tiles_n;
   int b = blockIdx.x;
   if constexpr (XR != 0) {
-    // XCD x = b % 8 runs ids x, x + 8, ...: ceil((ntiles - x) / 8) of them
-    const int q = ntiles >> 3, r = ntiles & 7, x = b & 7;
+    // XCD x = b % 8 runs ids x, x + 8, ...: ceil((total - x) / 8) of them
+    const int total = PART ? ntiles * p.splits : ntiles;
+    const int q = total >> 3, r = total & 7, x = b & 7;
     b = x * q + (x < r ? x : r) + (b >> 3);
   } else {
     if ((ntiles & 7) == 0) b = (b & 7) * (ntiles >> 3) + (b >> 3);
+  }
+  // split K: the tiles of one K range follow each other, so an XCD's share
+  // re-reads few columns of x; kbase..kbase + klen are this workgroup's k
+  int split = 0, kbase = 0, klen = p.k;
+  if constexpr (PART) {
+    static_assert(XR != 0 && NB == 1, "split K: one matrix, the XCD ranges of any count");
+    split = b / ntiles;
+    b -= split * ntiles;
+    const int steps = (p.k + 63) >> 6, per = (steps + p.splits - 1) / p.splits;
+    kbase = split * per * 64;
+    klen = p.k - kbase < per * 64 ? p.k - kbase : per * 64;
+    if (klen <= 0) klen = 0, kbase = 0;  // an empty range writes zeros
   }
   // inside the range: groups of group_m m-blocks, m fastest within a group
   const int per_group = p.group_m * p.tiles_n;
@@ -251,16 +268,16 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
   const int nrows_b = p.n - n0 < BN ? p.n - n0 : BN;
 
   constexpr int EB = I8 ? 1 : static_cast<int>(sizeof(TB));  // bytes per B element in memory
-  const rsrc_t rx = make_rsrc(static_cast<const TB*>(p.x) + static_cast<int64_t>(m0) * p.xs,
-                              static_cast<uint32_t>(((nrows_x - 1) * p.xs + p.k) * sizeof(TB)));
+  const rsrc_t rx = make_rsrc(static_cast<const TB*>(p.x) + static_cast<int64_t>(m0) * p.xs + kbase,
+                              static_cast<uint32_t>(((nrows_x - 1) * p.xs + klen) * sizeof(TB)));
   rsrc_t rb[NB];
-  rb[0] = make_rsrc(static_cast<const uint8_t*>(p.b0) + static_cast<int64_t>(n0) * p.bs * EB,
-                    static_cast<uint32_t>(((nrows_b - 1) * p.bs + p.k) * EB));
+  rb[0] = make_rsrc(static_cast<const uint8_t*>(p.b0) + (static_cast<int64_t>(n0) * p.bs + kbase) * EB,
+                    static_cast<uint32_t>(((nrows_b - 1) * p.bs + klen) * EB));
   if constexpr (NB == 2)
-    rb[1] = make_rsrc(static_cast<const uint8_t*>(p.b1) + static_cast<int64_t>(n0) * p.bs * EB,
-                      static_cast<uint32_t>(((nrows_b - 1) * p.bs + p.k) * EB));
+    rb[1] = make_rsrc(static_cast<const uint8_t*>(p.b1) + (static_cast<int64_t>(n0) * p.bs + kbase) * EB,
+                      static_cast<uint32_t>(((nrows_b - 1) * p.bs + klen) * EB));
 
-  const int nk = (p.k + 63) >> 6;
+  const int nk = (klen + 63) >> 6;
   // DMA lane maps (16-bit tiles).  Instruction j of wave w fills the 1 KiB
   // at tile offset 1024 (NW j + w): lane l writes physical chunk l % 8 of row
   // 8 (NW j + w) + l / 8, so it loads the logical chunk the swizzle keeps
@@ -290,7 +307,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
       b_col[j] = 8 * c;
     }
   }
-  const int kfull = p.k >> 6;  // steps whose 64 columns are all inside k
+  const int kfull = klen >> 6;  // steps whose 64 columns are all inside k
 
   // Issues the DMA of K step kt into stage I.  Columns at or past k read 0.
   auto issue = [&](auto I, int kt) {
@@ -301,7 +318,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
       const uint32_t kb = static_cast<uint32_t>(kt * 64 * sizeof(TB));
       const uint32_t dst = st + 1024u * (NW * j + wave);
       if (full) dma16(rx, a_goff[j], kb, dst);
-      else dma16(rx, kt * 64 + a_col[j] < p.k ? a_goff[j] + kb : kOob, 0, dst);
+      else dma16(rx, kt * 64 + a_col[j] < klen ? a_goff[j] + kb : kOob, 0, dst);
     }
 #pragma unroll
     for (int bi = 0; bi < NB; ++bi) {
@@ -310,7 +327,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
         const uint32_t kb = static_cast<uint32_t>(kt * 64 * EB);
         const uint32_t dst = st + C::A_BYTES + bi * C::B_BYTES + 1024u * (NW * j + wave);
         if (full) dma16(rb[bi], b_goff[j], kb, dst);
-        else dma16(rb[bi], kt * 64 + b_col[j] < p.k ? b_goff[j] + kb : kOob, 0, dst);
+        else dma16(rb[bi], kt * 64 + b_col[j] < klen ? b_goff[j] + kb : kOob, 0, dst);
       }
     }
   };
@@ -601,6 +618,35 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
   // 32x32 tile is transposed: lane l, register r -> x row l % 32, output
   // column (r & 3) + 4 (l / 32) + 8 (r / 4).  Registers 4g .. 4g + 3 are four
   // consecutive columns of one row: one 8-byte store (16 bytes for fp32).
+  if constexpr (PART) {
+    // the fp32 sums of this K range; rows of n % 4 == 0 floats are 16-byte aligned
+    float* base = p.part + (static_cast<int64_t>(split) * p.rows + m0) * p.n + n0;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int nl = wn * FN * 32 + 32 * j + 4 * static_cast<int>(h) + 8 * g;
+        if (nl >= nrows_b) continue;
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+          const int ml = wm * FM * 32 + 32 * i + static_cast<int>(lrow);
+          if (ml >= nrows_x) continue;
+          float* o = base + static_cast<int64_t>(ml) * p.n + nl;
+          const f32x16& a = acc[0][i][j];
+          if ((p.n & 3) == 0) {
+            *reinterpret_cast<u32x4*>(o) =
+                u32x4{as_u32(a[4 * g]), as_u32(a[4 * g + 1]), as_u32(a[4 * g + 2]), as_u32(a[4 * g + 3])};
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              if (nl + e < nrows_b) o[e] = a[4 * g + e];
+            }
+          }
+        }
+      }
+    }
+    return;
+  }
   const bool vec_out = (p.os & 3) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
 #pragma unroll
   for (int j = 0; j < FN; ++j) {
@@ -618,7 +664,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
             if (nl + e < nrows_b) bz[e] = load_dyn(p.bias, n + e, p.bdt);
           }
         }
-      } else if constexpr (EPI != EPI_SILU) {
+      } else if constexpr (EPI != EPI_SILU && !PART) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
           if (nl + e < nrows_b) {

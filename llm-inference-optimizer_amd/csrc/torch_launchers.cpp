@@ -145,6 +145,13 @@ std::vector<int64_t> with_last(at::IntArrayRef s, int64_t last) {
 
 void* ptr(const at::Tensor& t) { return t.data_ptr(); }
 
+// A call's scratch memory: `bytes` from torch's allocator on the current
+// stream (the launch stream, so its reuse is ordered after the call's kernels;
+// a captured graph keeps it in its pool), or an undefined tensor for 0.
+at::Tensor workspace(int64_t bytes, const at::Tensor& like) {
+  return bytes > 0 ? at::empty({bytes}, like.options().dtype(at::kByte)) : at::Tensor();
+}
+
 // ------------------------------------------------------------------ RMSNorm
 
 at::Tensor rmsnorm(const at::Tensor& x, const at::Tensor& weight, double eps) {
@@ -299,10 +306,11 @@ at::Tensor linear16(const at::Tensor& x, const at::Tensor& weight, const c10::op
     const int64_t xs = M > 1 ? x2.stride(0) : K;
     const int64_t ws = N > 1 ? w.stride(0) : K;
     Launch l(dev);
+    const at::Tensor work = workspace(mi355_linear16_workspace(M, K, N), x);
     check("mi355_linear16_fwd",
-          mi355_linear16_fwd(ptr(x2), ptr(w), has_bias ? ptr(b) : nullptr, ptr(out), M, K, N, xs, ws, N,
-                             code_of(x.scalar_type()), has_bias ? code_of(b.scalar_type()) : 0, code_of(odt),
-                             l.stream));
+          mi355_linear16_ws_fwd(ptr(x2), ptr(w), has_bias ? ptr(b) : nullptr, ptr(out), M, K, N, xs, ws, N,
+                                code_of(x.scalar_type()), has_bias ? code_of(b.scalar_type()) : 0, code_of(odt),
+                                work.defined() ? ptr(work) : nullptr, work.defined() ? work.numel() : 0, l.stream));
   }
   return out.reshape(with_last(x.sizes(), N));
 }
@@ -340,10 +348,12 @@ at::Tensor w8a16_linear(const at::Tensor& x, const at::Tensor& w_q, const at::Te
     const int64_t xs = M > 1 ? x2.stride(0) : K;
     const int64_t ws = N > 1 ? q.stride(0) : K;
     Launch l(dev);
+    const at::Tensor work = workspace(mi355_w8a16_linear_workspace(M, K, N), x);
     check("mi355_w8a16_linear_fwd",
-          mi355_w8a16_linear_fwd(ptr(x2), ptr(q), ptr(s), has_bias ? ptr(b) : nullptr, ptr(out), M, K, N, xs, ws, N,
-                                 code_of(x.scalar_type()), code_of(s.scalar_type()),
-                                 has_bias ? code_of(b.scalar_type()) : 0, code_of(odt), l.stream));
+          mi355_w8a16_linear_ws_fwd(ptr(x2), ptr(q), ptr(s), has_bias ? ptr(b) : nullptr, ptr(out), M, K, N, xs, ws, N,
+                                    code_of(x.scalar_type()), code_of(s.scalar_type()),
+                                    has_bias ? code_of(b.scalar_type()) : 0, code_of(odt),
+                                    work.defined() ? ptr(work) : nullptr, work.defined() ? work.numel() : 0, l.stream));
   }
   return out.reshape(with_last(x.sizes(), N));
 }

@@ -11,7 +11,7 @@
 // applied once to the fp32 accumulator, then the bias (fp32), then one
 // rounding to the output type.  Here scale and bias go through one fma.
 //
-// Four kernels, picked by the launcher:
+// Five kernels, picked by the launcher:
 //   w8a16_stream   rows <= 16 (decode; w8a16_stream.h), and 17 - 48 (49 -
 //                  64 for one matrix of at most 8 MB) where the small tiled
 //                  shapes do not pay (and the gate/up + SiLU-and-mul at 17 -
@@ -25,7 +25,10 @@
 //   tiled_gemm     more rows (prefill): the LDS-tiled MFMA GEMM of
 //                  tiled_gemm.h with int8 weights kept int8 in LDS and widened
 //                  after each LDS read, scale and bias in its epilogue.
-//   w8a16_generic  any k, stride or alignment the three above cannot take:
+//   split_k.h      one matrix from 17 rows, given a workspace, where the
+//                  output holds too few tiles for the CUs: the tiled GEMM
+//                  over ranges of K and a second pass that adds them.
+//   w8a16_generic  any k, stride or alignment the others cannot take:
 //                  one wave per (output feature, 4 rows of x), fp32 fma.
 //
 // And the quantiser of QuantizedLinearInt8.from_linear
@@ -55,6 +58,7 @@
 // traffic), so any k that is a multiple of 16 needs no remainder loop.  The
 // per-wave partial sums meet in LDS in a fixed order.
 #include "common.h"
+#include "split_k.h"
 #include "tiled_gemm.h"
 #include "w8a16_stream.h"
 
@@ -355,6 +359,26 @@ bool tiled_fits(const W8Params& p, bool) {
          static_cast<int64_t>((p.rows + 63) / 64) * ((p.n + 63) / 64) < (int64_t{1} << 31);
 }
 
+tiled::Params w8_tiled_params(const W8Params& p, const void* b1) {
+  tiled::Params tp{};
+  tp.x = p.x;
+  tp.b0 = p.q;
+  tp.b1 = b1;
+  tp.scale = p.scale;
+  tp.scale1 = p.scale2;
+  tp.bias = p.bias;
+  tp.out = p.out;
+  tp.rows = p.rows;
+  tp.k = p.k;
+  tp.n = p.n;
+  tp.xs = p.xs;
+  tp.bs = p.qs;
+  tp.os = p.os;
+  tp.sdt = p.sdt;
+  tp.bdt = p.bdt;
+  return tp;
+}
+
 // m-blocks per group of the tiled GEMM's tile order inside each XCD's range
 // (m fastest within a group).
 constexpr int kW8GroupM = 4;
@@ -374,22 +398,7 @@ int w8_tiled_cfg(const W8Params& p, hipStream_t s) {
     const int64_t ntiles = static_cast<int64_t>((p.rows + C::BM - 1) / C::BM) * ((p.n + C::BN - 1) / C::BN);
     if (ntiles % 8 != 0) return w8_tiled_cfg<T, TO, WGM, WGN, FM, FN, S, EPI, RING, WPE, 1>(p, s);
   }
-  tiled::Params tp{};
-  tp.x = p.x;
-  tp.b0 = p.q;
-  tp.b1 = EPI == tiled::EPI_SILU_W8 ? p.q2 : p.q;
-  tp.scale = p.scale;
-  tp.scale1 = p.scale2;
-  tp.bias = p.bias;
-  tp.out = p.out;
-  tp.rows = p.rows;
-  tp.k = p.k;
-  tp.n = p.n;
-  tp.xs = p.xs;
-  tp.bs = p.qs;
-  tp.os = p.os;
-  tp.sdt = p.sdt;
-  tp.bdt = p.bdt;
+  tiled::Params tp = w8_tiled_params(p, EPI == tiled::EPI_SILU_W8 ? p.q2 : p.q);
   tp.tiles_m = (p.rows + C::BM - 1) / C::BM;
   tp.tiles_n = (p.n + C::BN - 1) / C::BN;
   tp.group_m = tp.tiles_m < kW8GroupM ? tp.tiles_m : kW8GroupM;
@@ -529,12 +538,21 @@ int w8_tiled_small(const W8Params& p, hipStream_t s) {
 }
 
 template <typename T, typename TO, bool DUAL>
-int w8_typed(const W8Params& p, hipStream_t s, int cus) {
+int w8_typed(const W8Params& p, hipStream_t s, int cus, void* work = nullptr, int64_t work_bytes = 0) {
   const bool vec = p.k % 16 == 0 && p.qs % 16 == 0 && p.xs % 8 == 0 && aligned16(p.x) && aligned16(p.q) &&
                    (!DUAL || aligned16(p.q2));
   if (!vec) {
     const int64_t waves = static_cast<int64_t>(p.n) * ((p.rows + kGenRows - 1) / kGenRows);
     return launch_w8(w8a16_generic<T, TO, DUAL>, dim3(static_cast<unsigned>((waves + 3) / 4)), dim3(256), 0, p, s);
+  }
+  // One matrix of at least 17 rows whose output holds too few tiles for the
+  // CUs: split K (split_k.h has the figures), where the plan predicts it
+  // faster than the kernels below.
+  if constexpr (!DUAL) {
+    const tiled::SplitPlan sp = tiled::split_plan(p.rows, p.k, p.n, 1, cus);
+    if (sp.tile >= 0 && work != nullptr && work_bytes >= tiled::split_bytes(sp, p.rows, p.n) && tiled_fits(p, DUAL))
+      return tiled::split_k_launch<T, tiled::B_I8, TO, tiled::EPI_W8>(w8_tiled_params(p, p.q), sp,
+                                                                       static_cast<float*>(work), s);
   }
   // Up to 16 rows, but 9 - 16 rows of wide outputs with 2048 < k < 3072
   // (w8a16_skinny there; at k >= 3072 the stream kernel's 16-row workgroups
@@ -586,16 +604,16 @@ int w8_typed(const W8Params& p, hipStream_t s, int cus) {
 
 int w8a16_launch(const void* x, const void* q, const void* scale, const void* bias, void* out, int rows, int k,
                  int n, int64_t xs, int64_t qs, int64_t os, int x_dtype, int scale_dtype, int bias_dtype,
-                 int out_dtype, hipStream_t stream) {
+                 int out_dtype, void* work, int64_t work_bytes, hipStream_t stream) {
   int cus = 0;
   const int st = compute_units(&cus);
   if (st != MI355_OK) return st;
   const W8Params p{x, q, scale, bias, out, rows, k, n, xs, qs, os, scale_dtype, bias ? bias_dtype : -1, nullptr,
                    nullptr};
-  if (x_dtype == MI355_F16 && out_dtype == MI355_F16) return w8_typed<F16, F16, false>(p, stream, cus);
-  if (x_dtype == MI355_F16 && out_dtype == MI355_F32) return w8_typed<F16, F32, false>(p, stream, cus);
-  if (x_dtype == MI355_BF16 && out_dtype == MI355_BF16) return w8_typed<BF16, BF16, false>(p, stream, cus);
-  if (x_dtype == MI355_BF16 && out_dtype == MI355_F32) return w8_typed<BF16, F32, false>(p, stream, cus);
+  if (x_dtype == MI355_F16 && out_dtype == MI355_F16) return w8_typed<F16, F16, false>(p, stream, cus, work, work_bytes);
+  if (x_dtype == MI355_F16 && out_dtype == MI355_F32) return w8_typed<F16, F32, false>(p, stream, cus, work, work_bytes);
+  if (x_dtype == MI355_BF16 && out_dtype == MI355_BF16) return w8_typed<BF16, BF16, false>(p, stream, cus, work, work_bytes);
+  if (x_dtype == MI355_BF16 && out_dtype == MI355_F32) return w8_typed<BF16, F32, false>(p, stream, cus, work, work_bytes);
   set_error("mi355_w8a16_linear_fwd: unsupported dtype pair (x=%d, out=%d)", x_dtype, out_dtype);
   return MI355_ERR_UNSUPPORTED;
 }
