@@ -1,7 +1,7 @@
 // C ABI entry points (include/mi355_fused.h): argument validation, the
 // per-thread error message and the per-device CU-count cache.  Kernels and
 // their launchers live in rmsnorm.hip, silu_mul.hip, gate_up_silu.hip,
-// w8a16.hip and linear16.hip.
+// w8a16.hip, quantize_int8.hip and linear16.hip.
 #include <atomic>
 #include <cstdarg>
 #include <cstdio>

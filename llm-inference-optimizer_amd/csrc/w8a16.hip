@@ -1,6 +1,6 @@
-// Weight-only int8 linear (W8A16), the int8 gate/up projections fused with
-// SiLU-and-mul, and the int8 weight quantiser for gfx950, with their
-// launchers.
+// Weight-only int8 linear (W8A16) and the int8 gate/up projections fused with
+// SiLU-and-mul for gfx950, with their launchers (the weight quantiser:
+// quantize_int8.hip).
 //
 //   out[m, n] = round(acc * scale[n] + bias[n]),  acc = sum_k x[m, k] * q[n, k]
 //
@@ -30,12 +30,6 @@
 //                  over ranges of K and a second pass that adds them.
 //   w8a16_generic  any k, stride or alignment the others cannot take:
 //                  one wave per (output feature, 4 rows of x), fp32 fma.
-//
-// And the quantiser of QuantizedLinearInt8.from_linear
-// (src/quantization/int8.py:45-50), one wave per weight row:
-//   amax = max_k |w|,  scale = max(amax / 127, 1e-8),
-//   q = clamp(rint(w / scale), -127, 127)   (IEEE fp32 division, ties to even)
-// which is bit-identical to the reference's torch expression.
 //
 // Skinny operand layout.  The 16x16x32 MFMA's B operand gives lane l column
 // n = l % 16 and k-group l / 16 (8 consecutive k).  Each lane loads 16 int8
@@ -234,44 +228,6 @@ __global__ __launch_bounds__(256) void w8a16_generic(const W8Params p) {
       if constexpr (DUAL) w8_store_silu<TO>(p, m0 + i, n, s[0], s[NQ - 1]);
       else w8_store<TO>(p, m0 + i, n, s[0]);
     }
-  }
-}
-
-// --------------------------------------------------------------- quantiser
-
-template <typename TW>
-__global__ __launch_bounds__(256) void quantize_int8_rows(const void* __restrict__ w, int8_t* __restrict__ q,
-                                                          float* __restrict__ scale, int64_t n, int k, int64_t ws,
-                                                          int64_t qs) {
-  const int lane = threadIdx.x & 63;
-  const int64_t r = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-  if (r >= n) return;
-  float amax = 0.f;
-  for (int c = lane; c < k; c += 64) amax = __builtin_fmaxf(amax, __builtin_fabsf(load_elem<TW>(w, r * ws + c)));
-  // max is exact and order-free; the symmetric butterfly leaves it in every lane
-  amax = __builtin_fmaxf(amax, dpp_f32<0xb1>(amax));
-  amax = __builtin_fmaxf(amax, dpp_f32<0x4e>(amax));
-  amax = __builtin_fmaxf(amax, dpp_f32<0x141>(amax));
-  amax = __builtin_fmaxf(amax, dpp_f32<0x140>(amax));
-  {
-    const uint32_t b = as_u32(amax);
-    auto s = __builtin_amdgcn_permlane16_swap(b, b, false, false);
-    const uint32_t lo = s[0], hi = s[1];
-    amax = __builtin_fmaxf(as_f32(lo), as_f32(hi));
-  }
-  {
-    const uint32_t b = as_u32(amax);
-    auto s = __builtin_amdgcn_permlane32_swap(b, b, false, false);
-    const uint32_t lo = s[0], hi = s[1];
-    amax = __builtin_fmaxf(as_f32(lo), as_f32(hi));
-  }
-  float sc = amax / 127.0f;  // IEEE division (HIP's default for fp32 '/')
-  if (sc < 1e-8f) sc = 1e-8f;
-  if (lane == 0) scale[r] = sc;
-  for (int c = lane; c < k; c += 64) {
-    float v = __builtin_rintf(load_elem<TW>(w, r * ws + c) / sc);
-    v = __builtin_fminf(__builtin_fmaxf(v, -127.0f), 127.0f);
-    q[r * qs + c] = static_cast<int8_t>(static_cast<int>(v));
   }
 }
 
@@ -631,21 +587,6 @@ int gate_up_silu_w8a16_launch(const void* x, const void* qg, const void* qu, con
   if (x_dtype == MI355_BF16 && out_dtype == MI355_F32) return w8_typed<BF16, F32, true>(p, stream, cus);
   set_error("mi355_gate_up_silu_w8a16_fwd: unsupported dtype pair (x=%d, out=%d)", x_dtype, out_dtype);
   return MI355_ERR_UNSUPPORTED;
-}
-
-int quantize_int8_launch(const void* w, void* q, void* scale, int64_t n, int k, int64_t ws, int64_t qs, int w_dtype,
-                         hipStream_t stream) {
-  const unsigned grid = static_cast<unsigned>((n + 3) / 4);
-  void* args[] = {const_cast<void**>(&w), &q, &scale, &n, &k, &ws, &qs};
-  const void* kern = nullptr;
-  if (w_dtype == MI355_F32) kern = reinterpret_cast<const void*>(quantize_int8_rows<F32>);
-  else if (w_dtype == MI355_F16) kern = reinterpret_cast<const void*>(quantize_int8_rows<F16>);
-  else if (w_dtype == MI355_BF16) kern = reinterpret_cast<const void*>(quantize_int8_rows<BF16>);
-  if (!kern) {
-    set_error("mi355_quantize_int8_fwd: unsupported weight dtype %d", w_dtype);
-    return MI355_ERR_UNSUPPORTED;
-  }
-  return hip_status(hipLaunchKernel(kern, dim3(grid), dim3(256), args, 0, stream), "quantize_int8 launch");
 }
 
 }  // namespace mi355
