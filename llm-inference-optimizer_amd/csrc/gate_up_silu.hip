@@ -52,6 +52,7 @@
 // j < 4, of column l % 16.
 #include "common.h"
 #include "tiled_gemm.h"
+#include "tiled_plan.h"
 #include "w8a16_stream.h"
 
 // Launch shapes (split-K waves, weight row groups, K steps in flight per
@@ -237,18 +238,11 @@ int gate_up_shape(const GateUpParams& p, hipStream_t s) {
 // (m fastest within a group).
 constexpr int kGuGroupM = 4;
 
-template <typename T, typename TO, int WGM, int WGN, int FM, int FN, int S, int RING = 0, int XR = 0>
+// S / SB: LDS stages of x / of the weights (tiled_gemm.h).
+template <typename T, typename TO, int WGM, int WGN, int FM, int FN, int S, int RING = 0, int SB = S>
 int gate_up_tiled_cfg(const GateUpParams& p, hipStream_t s) {
-  using C = tiled::Cfg<T, tiled::B_16, TO, WGM, WGN, FM, FN, tiled::EPI_SILU, S>;
+  using C = tiled::Cfg<T, tiled::B_16, TO, WGM, WGN, FM, FN, tiled::EPI_SILU, S, SB>;
   static_assert(C::LDS <= 160 * 1024, "LDS per workgroup");
-  // a tile count that is not a multiple of 8: the instantiation with
-  // contiguous tile ranges per XCD for any count (XR = 1; 1.5B at 384 rows
-  // 34.7 -> 29.7 us, at 1400 rows 92.5 -> 87.3 us, 7B at 1792 rows 435.8 ->
-  // 412.3 us)
-  if constexpr (XR == 0) {
-    const int64_t ntiles = static_cast<int64_t>((p.rows + C::BM - 1) / C::BM) * ((p.n_out + C::BN - 1) / C::BN);
-    if (ntiles % 8 != 0) return gate_up_tiled_cfg<T, TO, WGM, WGN, FM, FN, S, RING, 1>(p, s);
-  }
   tiled::Params tp{};
   tp.x = p.x;
   tp.b0 = p.wg;
@@ -268,103 +262,69 @@ int gate_up_tiled_cfg(const GateUpParams& p, hipStream_t s) {
   void* args[] = {&tp};
   // all LDS is static (no dynamic shared memory)
   return hip_status(hipLaunchKernel(reinterpret_cast<const void*>(tiled::tiled_gemm<T, tiled::B_16, TO, WGM, WGN, FM, FN,
-                                                                                      tiled::EPI_SILU, S, RING, 0, XR>),
+                                                                                      tiled::EPI_SILU, S, RING, 0,
+                                                                                      SB>),
                                     dim3(static_cast<unsigned>(tp.tiles_m * tp.tiles_n)), dim3(C::BLOCK), args, 0, s),
                     "gate_up_silu tiled launch");
 }
 
-// Tiled launch shapes from sweeps on MI355X (Qwen2.5-1.5B and 7B MLPs at
-// 16 - 64, 128 and 384 - 4096 rows): up to 32 rows 32 x 64 output tiles (2
-// waves) or, for n_out > 10000, 32 x 128 (4 waves); up to 64 rows 64 x 64 (4
-// waves; n_out > 10000 keeps the next shape); up to 128 rows 128 x 64 (4
-// waves, 4 stages) or, for n_out > 10000, 128 x 128 (8 waves, 3 stages); more
-// rows by the round count below (1.5B, 256 rows 37.9 -> 27.8 us, 384 rows
-// 48.1 -> 35.0 us, 768 rows 58.1 -> 48.7 us, 4096 rows 251 -> 233 us; 7B, 256
-// rows 118 -> 97 us, 2048 rows 518 -> 469 us).
-// The small shapes run 4 stages.  Descriptors span at most 256 rows of x and
-// 128 weight rows, each below 2^31 bytes.
+// Tiles from 33 rows on (tiled_plan.h): 64 x 64 (4 waves, 72 KiB of LDS, two
+// workgroups per CU), 128 x 64 (4 waves, 80 KiB, two per CU), 128 x 128, 192
+// x 128 and 256 x 128 (8 waves of 64, 96 or 128 x 32) on the sub-step ring,
+// and 256 x 64 (8 waves) in the step pipeline.  The ring's 128 x 64, 192 x
+// 128 and 256 x 128 keep 2 stages of x and 3 of the weights: the weights miss
+// L2 where x hits it, and a step's copy of them issued only one step ahead
+// arrived late (2 stages of both -> 2 / 3, 7B: 256 rows 94.8 -> 84.8 us on
+// 256 x 128, 512 rows 190.0 -> 146.2 on 128 x 64; 1.5B, 1000 rows 71.3 ->
+// 63.5 on 192 x 128).
+// Against the shapes and rounds rule before: 1.5B 389 rows 42.7 -> 32.9 us,
+// 7B 512 rows 164 -> 137, 0.5B 128 rows 11.2 -> 7.8, 14B 64 rows 90.6 -> 56.8.
+constexpr tiled::ShapeCost kGateUpCost[] = {{64, 64, 2, 1.7, {0.328, 0.551, 0}, 0.055, 0.101, 0},
+                                            {128, 64, 2, 3.6, {0.347, 0.715, 0}, 0.130, 0.038, 1.5},
+                                            {128, 128, 1, 1.6, {0.655, 0, 0}, 0.277, 0.035, 2.7},
+                                            {192, 128, 1, 1.3, {0.772, 0, 0}, 0.405, 0.007, 6.6},
+                                            {256, 128, 1, 1.4, {0.889, 0, 0}, 0.650, 0, 8.6},
+                                            {256, 64, 1, 0.1, {0.516, 0, 0}, 0.261, 0.068, 5.2}};
+
+template <typename T, typename TO>
+int gate_up_shape_launch(const GateUpParams& p, int shape, hipStream_t s) {
+  switch (shape) {
+    case 0: return gate_up_tiled_cfg<T, TO, 2, 2, 1, 1, 3, 1>(p, s);
+    case 1: return gate_up_tiled_cfg<T, TO, 2, 2, 2, 1, 2, 1, 3>(p, s);
+    case 2: return gate_up_tiled_cfg<T, TO, 2, 4, 2, 1, 3, 1>(p, s);
+    case 3: return gate_up_tiled_cfg<T, TO, 2, 4, 3, 1, 2, 1, 3>(p, s);
+    case 4: return gate_up_tiled_cfg<T, TO, 2, 4, 4, 1, 2, 1, 3>(p, s);
+    default: return gate_up_tiled_cfg<T, TO, 4, 2, 2, 1, 3>(p, s);
+  }
+}
+
+// Up to 32 rows 32 x 64 output tiles (2 waves) or, for n_out > 10000, 32 x
+// 128 (4 waves), 4 stages; more rows by the plan, in one launch or in two on
+// column ranges (every output element sums its k products in the same order
+// either way).  Descriptors span at most 256 rows of x and 128 weight rows,
+// each below 2^31 bytes.
 template <typename T, typename TO>
 int gate_up_tiled(const GateUpParams& p, hipStream_t s) {
-  const bool wide = p.n_out > 10000;
   if (p.rows <= 32) {
-    if (wide) return gate_up_tiled_cfg<T, TO, 1, 4, 1, 1, 4>(p, s);  // 32 x 128, 4 waves
-    return gate_up_tiled_cfg<T, TO, 1, 2, 1, 1, 4>(p, s);            // 32 x 64, 2 waves
+    if (p.n_out > 10000) return gate_up_tiled_cfg<T, TO, 1, 4, 1, 1, 4>(p, s);  // 32 x 128, 4 waves
+    return gate_up_tiled_cfg<T, TO, 1, 2, 1, 1, 4>(p, s);                       // 32 x 64, 2 waves
   }
-  if (p.rows <= 64 && !wide) return gate_up_tiled_cfg<T, TO, 2, 2, 1, 1, 4>(p, s);  // 64 x 64, 4 waves
-  if (p.rows <= 128) {
-    if (p.n_out <= 10000) return gate_up_tiled_cfg<T, TO, 2, 2, 2, 1, 4>(p, s);
-    return gate_up_tiled_cfg<T, TO, 2, 4, 2, 1, 3>(p, s);
-  }
-  // More rows: the plan with the fewest weighted rounds of workgroups over
-  // the CUs, in units of one round of 256 x 64 tiles (8 waves, 3 stages).
-  // One shape for the whole output: 256 x 64; 128 x 64 (4 waves, the
-  // sub-step ring at 2 stages: 64 KiB of LDS, two workgroups per CU, each
-  // with its own barriers), 1.05 a round; 256 x 128 (8 waves of 128 x 32,
-  // the sub-step ring at 2 stages), which moves two thirds of 256 x 64's
-  // operand bytes per MFMA through the DMA and three quarters through LDS
-  // reads, 1.72 a round for twice the work.  Or a column split: whole rounds
-  // of 256 x 128 tiles over the leading columns, then the remaining columns
-  // in one round of the smallest tile that covers them in one -- 64 x 64 (4
-  // waves, 0.8), 128 x 64 (4 waves, 4 stages, 1.0), 128 x 64 on the ring
-  // (two per CU, 1.05) or 256 x 64 (1.0) -- so a last, thinly filled round
-  // of large tiles becomes a full round of small ones (1.5B, 1024 rows
-  // 80.5 -> 64.6 us).  The whole rounds are counted in tiles, not in
-  // 128-column blocks per round: with 6 row blocks, 3 rounds on 256 CUs hold
-  // 128 column blocks, where 3 x 42 blocks of whole columns per round left 4
-  // CUs idle each round and the rest too wide for one round of small tiles
-  // (7B, 1536 rows: 368 -> 355 us).  The split is two launches of one kernel on column
-  // ranges: every output element sums its k products in the same order
-  // either way.  Weights are the measured per-round times at Qwen2.5-1.5B
-  // and 7B shapes; ties keep the single launch, then 256 x 64.
   int cus = 0;
   const int st = compute_units(&cus);
   if (st != MI355_OK) return st;
-  const auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
-  const auto rounds = [&](int rows, int cols, int bm, int bn, int per_cu) {
-    return static_cast<double>(cdiv(cdiv(rows, bm) * cdiv(cols, bn), static_cast<int64_t>(cus) * per_cu));
-  };
-  const double c64 = rounds(p.rows, p.n_out, 256, 64, 1), c_small = 1.05 * rounds(p.rows, p.n_out, 128, 64, 2),
-               c128 = 1.72 * rounds(p.rows, p.n_out, 256, 128, 1);
-  const double single = c64 < c_small ? (c64 < c128 ? c64 : c128) : (c_small < c128 ? c_small : c128);
-
-  // 256 x 128 tiles (a ragged tile count gets XCD ranges, as every launch
-  // does: 1.5B at 768 rows, 210 tiles, 49.0 -> 46.3 us; at 1536 rows, 420
-  // tiles, 93.6 -> 90.5 us)
-  const auto big_tiles = [&](const GateUpParams& q) { return gate_up_tiled_cfg<T, TO, 2, 4, 4, 1, 2, 1>(q, s); };
-  // whole rounds of 256 x 128 tiles, and the 128-column blocks that fill
-  // them (a round need not end at a column boundary: the head launch's
-  // tiles fill its rounds in order)
-  const int64_t tiles_m = cdiv(p.rows, 256);
-  const int64_t full = cdiv(p.n_out, 128) * tiles_m / cus;
-  const int lead = static_cast<int>(full * cus / tiles_m * 128);  // columns in whole rounds
-  if (full >= 1 && lead > 0 && lead < p.n_out) {
-    const int rest = p.n_out - lead;
-    const auto one_round = [&](int bm, int bn, int per_cu) { return rounds(p.rows, rest, bm, bn, per_cu) <= 1.0; };
-    int shape = 0;
-    double rest_cost = 0.0;
-    if (one_round(64, 64, 1)) shape = 1, rest_cost = 0.8;
-    else if (one_round(128, 64, 1)) shape = 2, rest_cost = 1.0;
-    else if (one_round(128, 64, 2)) shape = 3, rest_cost = 1.05;
-    else if (one_round(256, 64, 1)) shape = 4, rest_cost = 1.0;
-    if (shape != 0 && 1.72 * static_cast<double>(full) + rest_cost < single) {
-      GateUpParams head = p, tail = p;
-      head.n_out = lead;
-      tail.n_out = rest;
-      const int64_t wskip = static_cast<int64_t>(lead) * p.ws * static_cast<int64_t>(sizeof(typename T::bits));
-      tail.wg = static_cast<const uint8_t*>(p.wg) + wskip;
-      tail.wu = static_cast<const uint8_t*>(p.wu) + wskip;
-      tail.out = static_cast<uint8_t*>(p.out) + static_cast<int64_t>(lead) * static_cast<int64_t>(sizeof(typename TO::bits));
-      const int r = big_tiles(head);
-      if (r != MI355_OK) return r;
-      if (shape == 1) return gate_up_tiled_cfg<T, TO, 2, 2, 1, 1, 4>(tail, s);
-      if (shape == 2) return gate_up_tiled_cfg<T, TO, 2, 2, 2, 1, 4>(tail, s);
-      if (shape == 3) return gate_up_tiled_cfg<T, TO, 2, 2, 2, 1, 2, 1>(tail, s);
-      return gate_up_tiled_cfg<T, TO, 4, 2, 2, 1, 3>(tail, s);
-    }
-  }
-  if (c64 == single) return gate_up_tiled_cfg<T, TO, 4, 2, 2, 1, 3>(p, s);
-  if (c_small == single) return gate_up_tiled_cfg<T, TO, 2, 2, 2, 1, 2, 1>(p, s);
-  return big_tiles(p);
+  const double wmb = 4e-6 * static_cast<double>(p.n_out) * p.k;
+  const tiled::TilePlan tp = tiled::plan_tiles(kGateUpCost, p.rows, p.n_out, p.k, wmb, cus, true);
+  if (tp.lead == 0) return gate_up_shape_launch<T, TO>(p, tp.shape, s);
+  GateUpParams head = p, tail = p;
+  head.n_out = tp.lead;
+  tail.n_out = p.n_out - tp.lead;
+  const int64_t wskip = static_cast<int64_t>(tp.lead) * p.ws * static_cast<int64_t>(sizeof(typename T::bits));
+  tail.wg = static_cast<const uint8_t*>(p.wg) + wskip;
+  tail.wu = static_cast<const uint8_t*>(p.wu) + wskip;
+  tail.out = static_cast<uint8_t*>(p.out) + static_cast<int64_t>(tp.lead) * static_cast<int64_t>(sizeof(typename TO::bits));
+  const int r = gate_up_shape_launch<T, TO>(head, tp.shape, s);
+  if (r != MI355_OK) return r;
+  return gate_up_shape_launch<T, TO>(tail, tp.tail, s);
 }
 
 template <typename T, typename TO>

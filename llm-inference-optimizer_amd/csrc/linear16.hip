@@ -116,9 +116,10 @@ tiled::Params l16_tiled_params(const L16Params& p) {
   return tp;
 }
 
-template <typename T, typename TO, int WGM, int WGN, int FM, int FN, int S, int RING = 0, int XR = 1>
+// S / SB: LDS stages of x / of the weights.
+template <typename T, typename TO, int WGM, int WGN, int FM, int FN, int S, int RING = 0, int SB = S>
 int l16_tiled_cfg(const L16Params& p, hipStream_t s) {
-  using C = tiled::Cfg<T, tiled::B_16, TO, WGM, WGN, FM, FN, tiled::EPI_LINEAR, S>;
+  using C = tiled::Cfg<T, tiled::B_16, TO, WGM, WGN, FM, FN, tiled::EPI_LINEAR, S, SB>;
   static_assert(C::LDS <= 160 * 1024, "LDS per workgroup");
   tiled::Params tp = l16_tiled_params(p);
   tp.tiles_m = (p.rows + C::BM - 1) / C::BM;
@@ -127,25 +128,30 @@ int l16_tiled_cfg(const L16Params& p, hipStream_t s) {
   void* args[] = {&tp};
   // all LDS is static (no dynamic shared memory)
   return hip_status(hipLaunchKernel(reinterpret_cast<const void*>(tiled::tiled_gemm<T, tiled::B_16, TO, WGM, WGN, FM, FN,
-                                                                                      tiled::EPI_LINEAR, S, RING, 0, XR>),
+                                                                                      tiled::EPI_LINEAR, S, RING, 0, SB>),
                                     dim3(static_cast<unsigned>(tp.tiles_m * tp.tiles_n)), dim3(C::BLOCK), args, 0, s),
                     "linear16 tiled launch");
 }
 
-// Unsplit tiles of more than 64 rows, by split_plan's predicted times: 64 x
-// 64 (4 waves, 4 stages), then on the sub-step ring 64 x 128 (4 stages), 128
-// x 128 (3), 256 x 128 and 256 x 256 (2).  (The rule before -- 64 x 64 below
-// 128 tiles of 128 x 128, else those in the step pipeline -- took 1.5B q/o
-// 1000 rows 12.6 us, now 11.2; 3B 16.9, now 12.9; the 14B q/o 333 rows 45.1,
-// now 36.8.)
+// Unsplit tiles of more than 64 rows, by split_plan's predicted times
+// (tiled_plan.h): 64 x 64 (4 waves, 4 stages) in the step pipeline, then on
+// the sub-step ring 128 x 64 (4 waves, 3 stages of x and 4 of the weights, two
+// workgroups per CU), 64 x 128 (8 waves, 4 stages), 128 x 128 (3 stages; or 2
+// of x and 3 of the weights, two per CU), 256 x 128 (3 and 4) and 256 x 256 (2
+// and 3).  (The rule before -- 64 x 64 below 128 tiles of 128 x 128, else
+// those in the step pipeline -- took 3B q/o at 1000 rows 16.9 us, now 12.9;
+// the 14B q/o at 333 rows 45.1, now 36.8; over the Qwen2.5-0.5B to 14B
+// projections at 72 - 4096 rows the plan takes 0.87 of its time.)
 template <typename T, typename TO>
 int l16_tiled(const L16Params& p, int shape, hipStream_t s) {
   switch (shape) {
     case 0: return l16_tiled_cfg<T, TO, 2, 2, 1, 1, 4>(p, s);
-    case 1: return l16_tiled_cfg<T, TO, 2, 4, 1, 1, 4, 1>(p, s);
-    case 2: return l16_tiled_cfg<T, TO, 2, 4, 2, 1, 3, 1>(p, s);
-    case 3: return l16_tiled_cfg<T, TO, 2, 4, 4, 1, 2, 1>(p, s);
-    default: return l16_tiled_cfg<T, TO, 2, 4, 4, 2, 2, 1>(p, s);
+    case 1: return l16_tiled_cfg<T, TO, 2, 2, 2, 1, 3, 1, 4>(p, s);
+    case 2: return l16_tiled_cfg<T, TO, 2, 4, 1, 1, 4, 1>(p, s);
+    case 3: return l16_tiled_cfg<T, TO, 2, 4, 2, 1, 3, 1>(p, s);
+    case 4: return l16_tiled_cfg<T, TO, 2, 4, 2, 1, 2, 1, 3>(p, s);
+    case 5: return l16_tiled_cfg<T, TO, 2, 4, 4, 1, 3, 1, 4>(p, s);
+    default: return l16_tiled_cfg<T, TO, 2, 4, 4, 2, 2, 1, 3>(p, s);
   }
 }
 
@@ -157,10 +163,10 @@ int l16_tiled(const L16Params& p, int shape, hipStream_t s) {
 template <typename T, typename TO>
 int l16_tiled_small(const L16Params& p, hipStream_t s) {
   if (p.rows <= 32) {
-    if (p.n > 10000) return l16_tiled_cfg<T, TO, 1, 4, 1, 1, 4, 0, 0>(p, s);
-    return l16_tiled_cfg<T, TO, 1, 2, 1, 1, 4, 0, 0>(p, s);
+    if (p.n > 10000) return l16_tiled_cfg<T, TO, 1, 4, 1, 1, 4>(p, s);
+    return l16_tiled_cfg<T, TO, 1, 2, 1, 1, 4>(p, s);
   }
-  return l16_tiled_cfg<T, TO, 2, 2, 1, 1, 4, 0, 0>(p, s);
+  return l16_tiled_cfg<T, TO, 2, 2, 1, 1, 4>(p, s);
 }
 
 template <typename T, typename TO>
@@ -217,9 +223,12 @@ int linear16_launch(const void* x, const void* w, const void* bias, void* out, i
 }
 
 int64_t split_workspace(int64_t rows, int64_t k, int64_t n, int weight_bytes) {
+  constexpr int64_t kMax = 0x7fffffff;
   int cus = 0;
-  if (rows <= 16 || k < 1 || n < 1 || compute_units(&cus) != MI355_OK) return 0;
-  return tiled::split_bytes(tiled::split_plan(rows, k, n, weight_bytes, cus), rows, n);
+  if (rows <= 16 || k < 1 || n < 1 || rows > kMax || k > kMax || n > kMax || compute_units(&cus) != MI355_OK) return 0;
+  return tiled::split_bytes(tiled::split_plan(static_cast<uint32_t>(rows), static_cast<uint32_t>(k),
+                                              static_cast<uint32_t>(n), weight_bytes, static_cast<uint32_t>(cus)),
+                            rows, n);
 }
 
 }  // namespace mi355

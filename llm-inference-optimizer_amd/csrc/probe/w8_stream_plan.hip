@@ -260,7 +260,8 @@ extern "C" __attribute__((visibility("default"))) void mi355_probe_gate_up16_str
 extern "C" __attribute__((visibility("default"))) long long mi355_probe_split_plan(long long rows, long long k,
                                                                                     long long n, int wb, int cus,
                                                                                     int* out4) {
-  const mi355::tiled::SplitPlan sp = mi355::tiled::split_plan(rows, k, n, wb, cus);
+  const mi355::tiled::SplitPlan sp = mi355::tiled::split_plan(
+      static_cast<uint32_t>(rows), static_cast<uint32_t>(k), static_cast<uint32_t>(n), wb, static_cast<uint32_t>(cus));
   out4[0] = sp.tile;
   out4[1] = sp.splits;
   out4[2] = sp.tile < 0 ? 0 : mi355::tiled::kSplitCost16[sp.tile].bm;

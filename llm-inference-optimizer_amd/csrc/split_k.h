@@ -28,6 +28,7 @@
 
 #include "common.h"
 #include "tiled_gemm.h"
+#include "tiled_plan.h"
 
 namespace mi355 {
 namespace tiled {
@@ -88,14 +89,12 @@ __global__ __launch_bounds__(256) void split_k_reduce(const Params p) {
 // (MB of weights).  Least-squares fits of a sweep on MI355X over the
 // Qwen2.5-0.5B to 14B down projections and square projections (896 - 5120
 // outputs, k 1536 - 18944) at 24 - 1500 rows, weights rotated through HBM:
-// mean error 2 - 5% per split tile, 5 - 12% per unsplit one; the plan's pick
-// is within 1.05x of the best measured shape on geometric average above 64
-// rows.
+// mean error 2 - 5% per tile.
 struct TileCost {
   int bm, bn;
   double c0, step, part, weight;
 };
-enum { SPLIT_TILES = 5, DIRECT_TILES = 5 };
+enum { SPLIT_TILES = 5 };
 // Split tiles: 32 x 128, 64 x 64, 64 x 128, 128 x 128, 256 x 256.
 constexpr TileCost kSplitCost16[SPLIT_TILES] = {
     {32, 128, 5.4, 0.256, 0.199, 0.113}, {64, 64, 5.0, 0.202, 0.288, 0.091},  {64, 128, 5.3, 0.310, 0.307, 0.087},
@@ -103,69 +102,68 @@ constexpr TileCost kSplitCost16[SPLIT_TILES] = {
 constexpr TileCost kSplitCost8[SPLIT_TILES] = {
     {32, 128, 6.4, 0.235, 0.249, 0.082}, {64, 64, 6.3, 0.226, 0.281, 0.053},  {64, 128, 6.8, 0.284, 0.320, 0.054},
     {128, 128, 8.9, 0.430, 0.226, 0.011}, {256, 256, 4.1, 1.659, 0.211, 0.005}};
-// Unsplit tiles: 64 x 64, 64 x 128, 128 x 128, 256 x 128, 256 x 256.
-constexpr TileCost kDirectCost16[DIRECT_TILES] = {{64, 64, 2.9, 0.206, 0, 0.155},
-                                                  {64, 128, 0.7, 0.300, 0, 0.242},
-                                                  {128, 128, 1.4, 0.389, 0, 0.255},
-                                                  {256, 128, 0, 0.791, 0, 0.408},
-                                                  {256, 256, 5.2, 1.149, 0, 0.277}};
-constexpr TileCost kDirectCost8[DIRECT_TILES] = {{64, 64, 6.5, 0.176, 0, 0.258},
-                                                 {64, 128, 5.6, 0.258, 0, 0.190},
-                                                 {128, 128, 6.3, 0.344, 0, 0.194},
-                                                 {256, 128, 5.3, 0.650, 0, 0.431},
-                                                 {256, 256, 11.8, 1.162, 0, 0.188}};
 // The weight-streaming kernel at 17 - 24, 25 - 32, 33 - 48 and 49 - 64 rows
 // (from 49 rows of more than 8 MB of int8 weights: the kernels that run
 // there): fixed us, us per MB of weights.
 constexpr double kStreamCost16[4][2] = {{3.1, 0.24}, {3.4, 0.29}, {4.1, 0.44}, {4.9, 0.52}};
 constexpr double kStreamCost8[4][2] = {{3.5, 0.36}, {4.1, 0.44}, {4.5, 0.69}, {4.9, 0.90}};
 
+// Whether 65 - 256 rows of an int8 product leave 32-row skinny tiles with split
+// K (w8a16.hip), which re-read the int8 weights per tile mostly from L2,
+// faster than unsplit tiles: tiny grids (fewer than 32 64 x 64 tiles: 1.5B
+// k/v at 96 - 256 rows, 6.4 vs 10.5 us) and narrow outputs (n < 2048) up to
+// 128 rows (1.5B down, 128 rows 30.7 vs 34.3 us).  Wider outputs and more
+// rows re-read too much (7B down, 96 rows 105.6 vs 82.8 us).
+inline bool w8_skinny_pays(uint32_t rows, uint32_t n) {
+  return rows <= 256 && (plan_cdiv(n, 64u) * plan_cdiv(rows, 64u) < 32 || (rows <= 128 && n < 2048));
+}
+
 struct SplitPlan {
   int tile;     // index into the split table; < 0: the unsplit kernels are faster
   int splits;   // K ranges, >= 2
   double cost;  // predicted us
-  int direct;   // the fastest unsplit tile (index into the direct table)
+  int direct;   // more than 64 rows: the fastest unsplit tile (index into kW8Cost / kL16Cost)
 };
 
 // The fastest split tile and count for [rows, k] x [n, k] (wb: bytes per
 // weight), against the fastest unsplit kernel at that size.  One workgroup
 // per CU: S = CUs / tiles, no more than 32, at least 4 K steps each, every
-// range with work.  Splitting has to win by 5% in the prediction; above 64
-// rows from k = 4096 on, where the fits of the unsplit tiles run low, it may
-// lose by 5% (int8 1.5B down, 1000 rows: predicted 44.7 against 44.3 us,
-// measured 41.9 against 49.2).
-inline SplitPlan split_plan(int64_t rows, int64_t k, int64_t n, int wb, int cus) {
-  const auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+// range with work.  Splitting has to win 3% and 1.5 us in the prediction (an
+// eager call also pays the second launch and the workspace on the host).
+inline SplitPlan split_plan(uint32_t rows, uint32_t k, uint32_t n, int wb, uint32_t cus) {
   const TileCost* sc = wb == 1 ? kSplitCost8 : kSplitCost16;
-  const TileCost* dc = wb == 1 ? kDirectCost8 : kDirectCost16;
-  const double wmb = static_cast<double>(n) * static_cast<double>(k) * wb * 1e-6;
-  const int64_t steps = cdiv(k, 64);
+  const double wmb = static_cast<double>(n) * k * wb * 1e-6;
   SplitPlan best{-1, 1, 1e30, 0};
   if (rows <= 16) return best;
-  double direct = 1e30;
-  for (int t = 0; t < DIRECT_TILES; ++t) {
-    const int64_t rounds = cdiv(cdiv(rows, dc[t].bm) * cdiv(n, dc[t].bn), cus);
-    const double c = dc[t].c0 + dc[t].step * static_cast<double>(steps * rounds) + dc[t].weight * wmb;
-    if (c < direct) direct = c, best.direct = t;
-  }
+  double direct;
   if (rows <= 64) {
     const int cls = rows <= 24 ? 0 : (rows <= 32 ? 1 : (rows <= 48 ? 2 : 3));
     const double* st = wb == 1 ? kStreamCost8[cls] : kStreamCost16[cls];
-    const double c = st[0] + st[1] * wmb;
-    if (c < direct) direct = c;
+    direct = st[0] + st[1] * wmb;
+  } else {
+    const TilePlan unsplit = wb == 1 ? plan_tiles(kW8Cost, rows, n, k, wmb, cus, false)
+                                     : plan_tiles(kL16Cost, rows, n, k, wmb, cus, false);
+    best.direct = unsplit.shape;
+    direct = unsplit.cost;
+    // 32-row skinny tiles, one K chain per workgroup (896 k 5.5 us, 1536 k
+    // 6.3, 3584 k 10.7, 4864 k 15.5)
+    if (wb == 1 && w8_skinny_pays(rows, n) && 3.0 + 0.0023 * k < direct) direct = 3.0 + 0.0023 * k;
   }
-  const double limit = direct * (rows > 64 && k >= 4096 ? 1.05 : 0.95);
+  const double limit = 0.97 * direct < direct - 1.5 ? 0.97 * direct : direct - 1.5;
+  const uint32_t steps = plan_cdiv(k, 64u);
   for (int t = 0; t < SPLIT_TILES; ++t) {
-    const int64_t tiles = cdiv(rows, sc[t].bm) * cdiv(n, sc[t].bn);
-    int64_t s = cus / tiles;
+    const double fixed = sc[t].c0 + sc[t].weight * wmb;
+    if (fixed >= limit) continue;
+    const uint32_t tiles = plan_cdiv(rows, static_cast<uint32_t>(sc[t].bm)) * plan_cdiv(n, static_cast<uint32_t>(sc[t].bn));
+    if (2 * tiles > cus) continue;
+    uint32_t s = cus / tiles;
     if (s > 32) s = 32;
     if (s > steps / 4) s = steps / 4;
     if (s < 2) continue;
-    const int64_t per = cdiv(steps, s);
-    s = cdiv(steps, per);
+    const uint32_t per = plan_cdiv(steps, s);
+    s = plan_cdiv(steps, per);
     if (s < 2) continue;
-    const double pmb = 8e-6 * static_cast<double>(s) * static_cast<double>(rows) * static_cast<double>(n);
-    const double c = sc[t].c0 + sc[t].step * static_cast<double>(per) + sc[t].part * pmb + sc[t].weight * wmb;
+    const double c = fixed + sc[t].step * per + sc[t].part * 8e-6 * s * rows * n;
     if (c < best.cost && c < limit) best = SplitPlan{t, static_cast<int>(s), c, best.direct};
   }
   return best;
@@ -187,7 +185,7 @@ int split_gemm_cfg(const Params& p0, hipStream_t s) {
   p.group_m = p.tiles_m < 4 ? p.tiles_m : 4;
   void* args[] = {&p};
   return hip_status(
-      hipLaunchKernel(reinterpret_cast<const void*>(tiled_gemm<T, BK, F32, WGM, WGN, FM, FN, EPI_PART, S, 1, 0, 1>),
+      hipLaunchKernel(reinterpret_cast<const void*>(tiled_gemm<T, BK, F32, WGM, WGN, FM, FN, EPI_PART, S, 1>),
                       dim3(static_cast<unsigned>(p.tiles_m * p.tiles_n * p.splits)), dim3(C::BLOCK), args, 0, s),
       "split-K launch");
 }

@@ -16,9 +16,13 @@
 // Decomposition.  A workgroup of WGM x WGN waves owns a BM x BN output tile
 // (BM = 32 FM WGM, BN = 32 FN WGN); each wave owns FM x FN 32x32 MFMA tiles
 // (of each B matrix).  K advances in steps of 64 columns through a ring of S
-// LDS stages filled by gfx950's global -> LDS DMA (buffer_load_dwordx4 ...
-// lds, 16 bytes per lane, no VGPR staging): step t + S - 1 is in flight while
-// step t computes.  Buffer descriptors end at the last valid element (rows
+// LDS stages of x and SB of the weights, filled by gfx950's global -> LDS DMA
+// (buffer_load_dwordx4 ... lds, 16 bytes per lane, no VGPR staging): step t +
+// S - 1 (SB - 1) is in flight while step t computes.  A copy takes 0.9 - 1 us
+// at a full chip, longer than one step of most tiles, and the weights' copies
+// come from HBM, so where LDS cannot hold a third whole stage it holds one of
+// the weights: 256 x 128 gate/up tiles with S = 2, SB = 3 take 15 - 25% less
+// time per step at 1 - 2 rounds than with SB = 2.  Buffer descriptors end at the last valid element (rows
 // past the matrix read 0); the K step enters through the scalar offset, and
 // only a final partial step redirects columns at or past k past the
 // descriptor, so any k that is a multiple of 16 (int8) or 8 (16-bit) works.
@@ -69,9 +73,9 @@
 //
 // Grid: one workgroup per tile, 1-D.  Consecutive workgroup ids land on
 // different XCDs (round robin over 8), so ids are remapped to give each XCD
-// a contiguous range of tiles, ordered in groups of group_m m-blocks, m
-// fastest: the x row blocks that share a weight block run on one XCD (tile
-// counts that are not a multiple of 8: see XR below).
+// a contiguous range of tiles (the first count mod 8 XCDs one tile longer),
+// ordered in groups of group_m m-blocks, m fastest: the x row blocks that
+// share a weight block run on one XCD.
 #pragma once
 
 #include <type_traits>
@@ -130,7 +134,7 @@ struct Params {
   int splits;   // EPI_PART: K ranges of ceil(steps / splits) 64-column steps each
 };
 
-template <typename T, int BK, typename TO, int WGM, int WGN, int FM, int FN, int EPI, int S>
+template <typename T, int BK, typename TO, int WGM, int WGN, int FM, int FN, int EPI, int S, int SB = S>
 struct Cfg {
   // BK: B's storage -- B_16 (x's 16-bit type) or B_I8 (int8, kept int8 in
   // LDS and widened after each LDS read).
@@ -142,20 +146,25 @@ struct Cfg {
   static constexpr int A_BYTES = BM * 128;             // 64 columns of 16-bit x per row
   static constexpr int B_ROW = I8 ? 64 : 128;          // bytes per B row per step in LDS
   static constexpr int B_BYTES = BN * B_ROW;
-  static constexpr int STAGE = A_BYTES + NB * B_BYTES;
-  static constexpr int LDS = S * STAGE;
+  static constexpr int LDS = S * A_BYTES + SB * NB * B_BYTES;  // S stages of x, SB of the weights
   // One DMA instruction moves 64 lanes x 16 bytes = 1 KiB: 8 rows of a 16-bit
   // tile, 16 rows of an int8 tile.
   static constexpr int AI = A_BYTES / 1024 / NW;  // A DMA instructions per wave per step
   static constexpr int BI = B_BYTES / 1024 / NW;  // B DMA instructions per wave per step and matrix
   static constexpr int P = AI + NB * BI;          // DMA instructions per wave per step
   static_assert(A_BYTES % (1024 * NW) == 0 && B_BYTES % (1024 * NW) == 0, "tile must split over the waves");
-  static_assert(S >= 2 && S <= 8, "2..8 stages");
-  static_assert(P * (S - 1) < 64, "vmcnt range");
+  // The operand with more stages is issued second in a step, so a wait for the
+  // next step leaves its younger copies, and WAIT instructions in all, in flight.
+  static constexpr int SMIN = S < SB ? S : SB, SMAX = S < SB ? SB : S;
+  static constexpr int WAIT = (SMIN - 2) * P + (S < SB ? NB * BI : (S > SB ? AI : 0));
+  static constexpr int FILL = S * AI + SB * NB * BI;  // instructions that fill every stage
+  static_assert(SMIN >= 2 && SMAX <= 10, "2..10 stages");
+  static_assert(FILL - P < 64, "vmcnt range");
 };
 
-// Stage I of the LDS ring (one LDS variable per stage).
-template <int I, int SZ> __device__ __forceinline__ uint8_t* stage_ptr() {
+// Stage I of an operand's LDS ring (one LDS variable per stage; OP 0: x, 1:
+// the weights).
+template <int OP, int I, int SZ> __device__ __forceinline__ uint8_t* stage_ptr() {
   __shared__ __attribute__((aligned(1024))) uint8_t st[SZ];
   return st;
 }
@@ -187,8 +196,8 @@ __device__ __forceinline__ void dma16(rsrc_t r, uint32_t voff, uint32_t soff, ui
 }
 
 // LDS byte address of stage I (the cast of the LDS variable itself folds to a constant).
-template <int I, int SZ> __device__ __forceinline__ uint32_t stage_addr() {
-  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)stage_ptr<I, SZ>()));
+template <int OP, int I, int SZ> __device__ __forceinline__ uint32_t stage_addr() {
+  return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr_t)stage_ptr<OP, I, SZ>()));
 }
 
 // Workgroup barrier that the compiler may not move memory accesses across.
@@ -213,19 +222,15 @@ constexpr int kMinWavesPerSimd = WPE > 0 ? WPE : 1;
 
 // WPE > 0 caps the registers of this configuration alone so that WPE waves fit
 // on each SIMD (a 192 x 128 tile of 8 waves at WPE = 4 fits in 128 VGPRs and
-// runs two workgroups per CU).  XR = 1 gives the XCDs contiguous tile ranges
-// when the tile count is not a multiple of 8 too (the first count mod 8 XCDs,
-// which receive one workgroup more, take ranges one tile longer); XR = 0
-// keeps the dispatch order for such counts.  (XR is a template argument so
-// that the configurations without it keep their code.)  The int8 B operand
+// runs two workgroups per CU).  The int8 B operand
 // is widened one sub-step ahead, into a second register set, after the
 // previous sub-step's MFMAs are issued, so the widening VALU work runs beside
 // the MFMAs instead of in front of them.
 template <typename T, int BK, typename TO, int WGM, int WGN, int FM, int FN, int EPI, int S, int RING = 0, int WPE = 0,
-          int XR = 0>
+          int SB = S>
 __global__ __launch_bounds__(64 * WGM * WGN)
 __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(const Params p) {
-  using C = Cfg<T, BK, TO, WGM, WGN, FM, FN, EPI, S>;
+  using C = Cfg<T, BK, TO, WGM, WGN, FM, FN, EPI, S, SB>;
   constexpr bool I8 = C::I8;
   using TB = typename T::bits;
   constexpr int NW = C::NW, BM = C::BM, BN = C::BN, NB = C::NB;
@@ -237,20 +242,15 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
   // Tile of this workgroup: contiguous ranges per XCD, m fastest.
   constexpr bool PART = EPI == EPI_PART;
   const int ntiles = p.tiles_m * p.tiles_n;
-  int b = blockIdx.x;
-  if constexpr (XR != 0) {
-    // XCD x = b % 8 runs ids x, x + 8, ...: ceil((total - x) / 8) of them
-    const int total = PART ? ntiles * p.splits : ntiles;
-    const int q = total >> 3, r = total & 7, x = b & 7;
-    b = x * q + (x < r ? x : r) + (b >> 3);
-  } else {
-    if ((ntiles & 7) == 0) b = (b & 7) * (ntiles >> 3) + (b >> 3);
-  }
+  // XCD x = id % 8 runs ids x, x + 8, ...: ceil((total - x) / 8) of them
+  const int total = PART ? ntiles * p.splits : ntiles;
+  const int xq = total >> 3, xr = total & 7, xcd = blockIdx.x & 7;
+  int b = xcd * xq + (xcd < xr ? xcd : xr) + (blockIdx.x >> 3);
   // split K: the tiles of one K range follow each other, so an XCD's share
   // re-reads few columns of x; kbase..kbase + klen are this workgroup's k
   int split = 0, kbase = 0, klen = p.k;
   if constexpr (PART) {
-    static_assert(XR != 0 && NB == 1, "split K: one matrix, the XCD ranges of any count");
+    static_assert(NB == 1, "split K: one matrix");
     split = b / ntiles;
     b -= split * ntiles;
     const int steps = (p.k + 63) >> 6, per = (steps + p.splits - 1) / p.splits;
@@ -309,9 +309,10 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
   }
   const int kfull = klen >> 6;  // steps whose 64 columns are all inside k
 
-  // Issues the DMA of K step kt into stage I.  Columns at or past k read 0.
-  auto issue = [&](auto I, int kt) {
-    const uint32_t st = stage_addr<decltype(I)::value, C::STAGE>();
+  // Issue the DMA of K step kt of x, or of the weights, into stage I of its
+  // ring.  Columns at or past k read 0.
+  auto issue_a = [&](auto I, int kt) {
+    const uint32_t st = stage_addr<0, decltype(I)::value, C::A_BYTES>();
     const bool full = kt < kfull;  // known true in the main loop (the compiler folds it)
 #pragma unroll
     for (int j = 0; j < C::AI; ++j) {
@@ -320,16 +321,29 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
       if (full) dma16(rx, a_goff[j], kb, dst);
       else dma16(rx, kt * 64 + a_col[j] < klen ? a_goff[j] + kb : kOob, 0, dst);
     }
+  };
+  auto issue_b = [&](auto I, int kt) {
+    const uint32_t st = stage_addr<1, decltype(I)::value, NB * C::B_BYTES>();
+    const bool full = kt < kfull;
 #pragma unroll
     for (int bi = 0; bi < NB; ++bi) {
 #pragma unroll
       for (int j = 0; j < C::BI; ++j) {
         const uint32_t kb = static_cast<uint32_t>(kt * 64 * EB);
-        const uint32_t dst = st + C::A_BYTES + bi * C::B_BYTES + 1024u * (NW * j + wave);
+        const uint32_t dst = st + bi * C::B_BYTES + 1024u * (NW * j + wave);
         if (full) dma16(rb[bi], b_goff[j], kb, dst);
         else dma16(rb[bi], kt * 64 + b_col[j] < klen ? b_goff[j] + kb : kOob, 0, dst);
       }
     }
+  };
+  // Fills the rings before the main loop: N stages of x, M of the weights.
+  auto prefill = [&](auto N, auto M) {
+    constexpr int n = decltype(N)::value, m = decltype(M)::value;
+    static_for([&](auto I) {
+      constexpr int i = decltype(I)::value;
+      if constexpr (i < n) { if (i < nk) issue_a(I, i); }
+      if constexpr (i < m) { if (i < nk) issue_b(I, i); }
+    }, std::make_index_sequence<(n > m ? n : m)>{});
   };
 
   f32x16 acc[NB][FM][FN];
@@ -360,7 +374,8 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
   };
   // LDS reads of sub-step s of one step (stage I) into f.
   auto read_sub = [&](auto I, Frags& f, int s) {
-    const uint8_t* abase = stage_ptr<decltype(I)::value, C::STAGE>();
+    const uint8_t* abase = stage_ptr<0, decltype(I)::value, C::A_BYTES>();
+    const uint8_t* bbase = stage_ptr<1, decltype(I)::value, NB * C::B_BYTES>();
 #pragma unroll
     for (int i = 0; i < FM; ++i) f.a[s][i] = lds_read16(abase, swz16(arow0 + 32 * i, 4 * h + s));
 #pragma unroll
@@ -368,9 +383,9 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
 #pragma unroll
       for (int j = 0; j < FN; ++j) {
         if constexpr (I8) {
-          if (s < BQ) f.b[bi][s][j] = lds_read16(abase + C::A_BYTES + bi * C::B_BYTES, swz8(brow0 + 32 * j, 2 * h + s));
+          if (s < BQ) f.b[bi][s][j] = lds_read16(bbase + bi * C::B_BYTES, swz8(brow0 + 32 * j, 2 * h + s));
         } else {
-          f.b[bi][s][j] = lds_read16(abase + C::A_BYTES + bi * C::B_BYTES, swz16(brow0 + 32 * j, 4 * h + s));
+          f.b[bi][s][j] = lds_read16(bbase + bi * C::B_BYTES, swz16(brow0 + 32 * j, 4 * h + s));
         }
       }
     }
@@ -436,7 +451,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
     // sub-step, runs the MFMAs of step t's sub-step s and issues the LDS reads
     // of step t + 1's sub-step s, so a wave's MFMAs never queue behind all of
     // its LDS reads (2-3% over all reads first).
-    static_assert(S >= 3, "the step pipeline needs 3 stages");
+    static_assert(S >= 3 && S == SB, "the step pipeline needs 3 stages, of both operands");
     Frags fr[2];
     // raw int8 pair q of a step's fragments as one [NB][FN] set
     auto raw_pair = [&](const Frags& f, int q, u32x4 (&out)[NB][FN]) {
@@ -451,9 +466,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
       raw_pair(f, (s >> 1) & (BQ - 1), raw);
       widen_into(raw, s, out);
     };
-    static_for([&](auto I) {
-      if (decltype(I)::value < nk) issue(I, decltype(I)::value);
-    }, std::make_index_sequence<S - 1>{});
+    prefill(std::integral_constant<int, S - 1>{}, std::integral_constant<int, S - 1>{});
     if (S - 2 < nk) wait_vmcnt<(S - 2) * C::P>();
     else wait_vmcnt<0>();
     wait_lgkmcnt0();
@@ -468,7 +481,10 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
     auto step = [&](auto I, auto GUARD, int t) {
       constexpr int ii = decltype(I)::value, si = ii % S, pi = ii % 2;
       constexpr bool guard = decltype(GUARD)::value;
-      if (!guard || t + S - 1 < nk) issue(std::integral_constant<int, (si + S - 1) % S>{}, t + S - 1);
+      if (!guard || t + S - 1 < nk) {
+        issue_a(std::integral_constant<int, (si + S - 1) % S>{}, t + S - 1);
+        issue_b(std::integral_constant<int, (si + S - 1) % S>{}, t + S - 1);
+      }
       const bool more = !guard || t + 1 < nk;
       if (more) {
         if (!guard || t + S - 1 < nk) wait_vmcnt<(S - 2) * C::P>();
@@ -521,15 +537,15 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
       u32x4 a[2][FM];
       u32x4 b[2][NB][FN];
     };
-    auto read_one = [&](auto I, Sub& f, int s) {
-      const uint8_t* abase = stage_ptr<decltype(I)::value, C::STAGE>();
+    auto read_one = [&](auto IA, auto IB, Sub& f, int s) {
+      const uint8_t* abase = stage_ptr<0, decltype(IA)::value, C::A_BYTES>();
 #pragma unroll
       for (int i = 0; i < FM; ++i) f.a[s & 1][i] = lds_read16(abase, swz16(arow0 + 32 * i, 4 * h + s));
 #pragma unroll
       for (int bi = 0; bi < NB; ++bi) {
 #pragma unroll
         for (int j = 0; j < FN; ++j) {
-          const uint8_t* bbase = abase + C::A_BYTES + bi * C::B_BYTES;
+          const uint8_t* bbase = stage_ptr<1, decltype(IB)::value, NB * C::B_BYTES>() + bi * C::B_BYTES;
           if constexpr (I8) {
             // raw pair q (sub-steps 2q, 2q + 1) read with sub-step q's A, a
             // sub-step or more before its first use: set q was last read
@@ -562,31 +578,36 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
       }
     };
     Sub rf;
-    static_for([&](auto I) {
-      if (decltype(I)::value < nk) issue(I, decltype(I)::value);
-    }, std::make_index_sequence<S>{});
-    if (S - 1 < nk) wait_vmcnt<(S - 1) * C::P>();
+    prefill(std::integral_constant<int, S>{}, std::integral_constant<int, SB>{});
+    if (C::SMAX - 1 < nk) wait_vmcnt<C::FILL - C::P>();
     else wait_vmcnt<0>();
     wait_lgkmcnt0();
     lds_barrier();
-    read_one(std::integral_constant<int, 0>{}, rf, 0);
+    read_one(std::integral_constant<int, 0>{}, std::integral_constant<int, 0>{}, rf, 0);
     if constexpr (WA) widen_into(rf.b[0], 0, wb[0]);
+    constexpr int UNROLL = lcm_c(S, SB);  // stage indices known at compile time
     auto rstep = [&](auto I, auto GUARD, int t) {
-      constexpr int si = decltype(I)::value % S;
+      constexpr int sa = decltype(I)::value % S, sb = decltype(I)::value % SB;
       constexpr bool guard = decltype(GUARD)::value;
       const bool more = !guard || t + 1 < nk;
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
         __builtin_amdgcn_sched_barrier(0);
         if (s < 3) {
-          read_one(std::integral_constant<int, si>{}, rf, s + 1);
+          read_one(std::integral_constant<int, sa>{}, std::integral_constant<int, sb>{}, rf, s + 1);
         } else if (more) {
-          if (!guard || t + S - 1 < nk) wait_vmcnt<(S - 2) * C::P>();
+          if (!guard || t + C::SMAX - 1 < nk) wait_vmcnt<C::WAIT>();
           else wait_vmcnt<0>();
           wait_lgkmcnt0();
           lds_barrier();
-          if (!guard || t + S < nk) issue(std::integral_constant<int, si>{}, t + S);
-          read_one(std::integral_constant<int, (si + 1) % S>{}, rf, 0);
+          if constexpr (S > SB) {
+            if (!guard || t + SB < nk) issue_b(std::integral_constant<int, sb>{}, t + SB);
+          }
+          if (!guard || t + S < nk) issue_a(std::integral_constant<int, sa>{}, t + S);
+          if constexpr (S <= SB) {
+            if (!guard || t + SB < nk) issue_b(std::integral_constant<int, sb>{}, t + SB);
+          }
+          read_one(std::integral_constant<int, (sa + 1) % S>{}, std::integral_constant<int, (sb + 1) % SB>{}, rf, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (WA) {
@@ -603,14 +624,15 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
       }
       __builtin_amdgcn_sched_barrier(0);
     };
-    // main loop: steps t0 .. t0 + S - 1 issue steps up to t0 + 2 S - 1 < kfull
-    for (; t0 + 2 * S - 1 < kfull; t0 += S) {
-      static_for([&](auto I) { rstep(I, std::false_type{}, t0 + decltype(I)::value); }, std::make_index_sequence<S>{});
+    // main loop: steps t0 .. t0 + UNROLL - 1 issue steps up to t0 + UNROLL + SMAX - 1 < kfull
+    for (; t0 + UNROLL + C::SMAX - 1 < kfull; t0 += UNROLL) {
+      static_for([&](auto I) { rstep(I, std::false_type{}, t0 + decltype(I)::value); },
+                 std::make_index_sequence<UNROLL>{});
     }
-    for (; t0 < nk; t0 += S) {
+    for (; t0 < nk; t0 += UNROLL) {
       static_for([&](auto I) {
         if (t0 + decltype(I)::value < nk) rstep(I, std::true_type{}, t0 + decltype(I)::value);
-      }, std::make_index_sequence<S>{});
+      }, std::make_index_sequence<UNROLL>{});
     }
   }
 

@@ -1,0 +1,106 @@
+// Which tile of tiled_gemm.h an unsplit product takes: a time model per tile
+// shape, fitted to measurements, and the shape (or pair of shapes on two
+// column ranges) it predicts fastest.  Host code, shared by the launchers.
+#pragma once
+
+#include <stdint.h>
+
+namespace mi355 {
+namespace tiled {
+
+// Predicted us of a [rows, k] x [cols, k] product on bm x bn tiles:
+//   c0 + round * rounds
+//      + (K steps of 64) * (full rounds * step[occ - 1] + last round's step
+//                           + load * tiles per CU)
+//      + weight * (MB of weights)
+// where a round is occ workgroups on every CU, and a last round that needs
+// only w of them per CU costs step[w - 1].  step[w - 1] is the part of a K
+// step that a CU with w workgroups waits for whether or not the others work;
+// `load` the part that follows the work of the whole chip (a fully loaded
+// chip lowers its clock: 1.8 GHz under these kernels at long prompts).  The
+// constants are least-squares fits (non-negative) to sweeps on MI355X over the
+// Qwen2.5-0.5B to 14B projections at 33 - 4096 rows, weights rotated through
+// HBM; mean error 3 - 7% per shape.
+// `round` is a tile's first loads and its epilogue, which nothing overlaps
+// where a CU holds one workgroup.
+struct ShapeCost {
+  int bm, bn, occ;
+  double c0, step[3], load, weight, round;
+};
+
+// (32-bit: the launchers bound rows, n, k and rows * n / 4 below 2^31.  The
+// plan runs in every call; with 64-bit divisions it cost one about 0.6 us, as
+// here, with constant tile sizes, one plan takes 0.02 us.)
+inline uint32_t plan_cdiv(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
+
+__attribute__((always_inline)) inline double shape_time(const ShapeCost& s, uint32_t rows, uint32_t cols, uint32_t k, double wmb, uint32_t cus) {
+  const uint32_t tiles = plan_cdiv(rows, static_cast<uint32_t>(s.bm)) * plan_cdiv(cols, static_cast<uint32_t>(s.bn));
+  const uint32_t slots = cus * static_cast<uint32_t>(s.occ);
+  const uint32_t full = tiles / slots, rest = tiles - full * slots;
+  double per_step = full * s.step[s.occ - 1] + s.load * tiles / cus;
+  if (rest > 0) per_step += s.step[(rest > cus) + (rest > 2 * cus)];
+  return s.c0 + s.round * (full + (rest > 0)) + plan_cdiv(k, 64u) * per_step + s.weight * wmb;
+}
+
+struct TilePlan {
+  int shape;        // the one shape, or the leading columns'
+  int lead;         // leading columns of a two-launch plan (0: one launch)
+  int tail;         // the remaining columns' shape (lead > 0)
+  double cost;      // predicted us
+};
+
+// The fastest single shape of the table; with `split`, also every pair of
+// launches that gives the leading columns whole rounds of one shape and the
+// remaining columns another, so a last, thinly filled round of large tiles
+// becomes a round of small ones.  (A round need not end at a column boundary:
+// the lead's tiles fill its rounds in order.)  wmb: MB of weights over all n
+// columns.
+template <int N>
+__attribute__((always_inline)) inline TilePlan plan_tiles(const ShapeCost (&table)[N], uint32_t rows, uint32_t n, uint32_t k, double wmb,
+                           uint32_t cus, bool split) {
+  TilePlan best{0, 0, 0, 1e30};
+#pragma unroll
+  for (int i = 0; i < N; ++i) {  // unrolled: the table's tile sizes become constants
+    const double c = shape_time(table[i], rows, n, k, wmb, cus);
+    if (c < best.cost) best = TilePlan{i, 0, 0, c};
+  }
+  if (!split) return best;
+  constexpr double kSecondLaunch = 1.7;  // us, of the same fits
+  for (int i = 0; i < N; ++i) {
+    const ShapeCost& s = table[i];
+    const uint32_t tiles_m = plan_cdiv(rows, static_cast<uint32_t>(s.bm));
+    const uint32_t slots = cus * static_cast<uint32_t>(s.occ);
+    const uint32_t full = plan_cdiv(n, static_cast<uint32_t>(s.bn)) * tiles_m / slots;
+    if (full < 1) continue;
+    const uint32_t lead = full * slots / tiles_m * static_cast<uint32_t>(s.bn);
+    if (lead == 0 || lead >= n) continue;
+    const double share = static_cast<double>(lead) / n;
+    const double head = shape_time(s, rows, lead, k, wmb * share, cus) + kSecondLaunch;
+    if (head >= best.cost) continue;
+    for (int j = 0; j < N; ++j) {
+      const double c = head + shape_time(table[j], rows, n - lead, k, wmb * (1 - share), cus);
+      if (c < best.cost) best = TilePlan{i, static_cast<int>(lead), j, c};
+    }
+  }
+  return best;
+}
+
+// One int8 matrix (w8a16.hip): 64 x 64, 64 x 128, 128 x 128, 192 x 128 (capped
+// at 128 registers, two per CU) and 32 x 64.
+constexpr ShapeCost kW8Cost[] = {{64, 64, 3, 6.1, {0.181, 0.262, 0.400}, 0.060, 0.050, 0},
+                                 {64, 128, 2, 2.8, {0.250, 0.432, 0}, 0.101, 0.026, 3.4},
+                                 {128, 128, 2, 3.2, {0.288, 0.557, 0}, 0.216, 0.001, 5.0},
+                                 {192, 128, 2, 3.0, {0.429, 0.761, 0}, 0.322, 0, 6.5},
+                                 {32, 64, 3, 5.5, {0.177, 0.262, 0.282}, 0.022, 0.052, 0}};
+// One 16-bit matrix (linear16.hip): 64 x 64, 128 x 64, 64 x 128, 128 x 128 (one
+// and two per CU), 256 x 128 and 256 x 256.
+constexpr ShapeCost kL16Cost[] = {{64, 64, 2, 2.0, {0.213, 0.368, 0}, 0, 0.138, 0.8},
+                                  {128, 64, 2, 3.2, {0.259, 0.533, 0}, 0.017, 0.126, 1.8},
+                                  {64, 128, 1, 1.2, {0.235, 0, 0}, 0.048, 0.164, 2.2},
+                                  {128, 128, 1, 1.5, {0.298, 0, 0}, 0.170, 0.126, 3.0},
+                                  {128, 128, 2, 2.4, {0.363, 0.433, 0}, 0.263, 0.085, 2.7},
+                                  {256, 128, 1, 0, {0.523, 0, 0}, 0.277, 0.011, 9.6},
+                                  {256, 256, 1, 0, {0.397, 0, 0}, 1.198, 0, 20.9}};
+
+}  // namespace tiled
+}  // namespace mi355

@@ -54,6 +54,7 @@
 #include "common.h"
 #include "split_k.h"
 #include "tiled_gemm.h"
+#include "tiled_plan.h"
 #include "w8a16_stream.h"
 
 namespace mi355 {
@@ -339,21 +340,12 @@ tiled::Params w8_tiled_params(const W8Params& p, const void* b1) {
 // (m fastest within a group).
 constexpr int kW8GroupM = 4;
 
+// S / SB: LDS stages of x / of the weights.
 template <typename T, typename TO, int WGM, int WGN, int FM, int FN, int S, int EPI = tiled::EPI_W8, int RING = 0,
-          int WPE = 0, int XR = 0>
+          int WPE = 0, int SB = S>
 int w8_tiled_cfg(const W8Params& p, hipStream_t s) {
-  using C = tiled::Cfg<T, tiled::B_I8, TO, WGM, WGN, FM, FN, EPI, S>;
+  using C = tiled::Cfg<T, tiled::B_I8, TO, WGM, WGN, FM, FN, EPI, S, SB>;
   static_assert(C::LDS <= 160 * 1024, "LDS per workgroup");
-  // A tile count that is not a multiple of 8 takes the instantiation that
-  // gives the XCDs contiguous tile ranges for any count (XR = 1; the
-  // multiples of 8 keep the other, whose code predates it).  Prefill row
-  // counts are mostly not powers of two: 1.5B gate/up at 1400 rows (770
-  // tiles of 128 x 128) 66.1 -> 58.3 us, 2900 rows 112.0 -> 103.8 us, 7B
-  // gate/up at 1100 rows 179.2 -> 174.9 us; the narrow outputs even.
-  if constexpr (XR == 0) {
-    const int64_t ntiles = static_cast<int64_t>((p.rows + C::BM - 1) / C::BM) * ((p.n + C::BN - 1) / C::BN);
-    if (ntiles % 8 != 0) return w8_tiled_cfg<T, TO, WGM, WGN, FM, FN, S, EPI, RING, WPE, 1>(p, s);
-  }
   tiled::Params tp = w8_tiled_params(p, EPI == tiled::EPI_SILU_W8 ? p.q2 : p.q);
   tp.tiles_m = (p.rows + C::BM - 1) / C::BM;
   tp.tiles_n = (p.n + C::BN - 1) / C::BN;
@@ -361,112 +353,66 @@ int w8_tiled_cfg(const W8Params& p, hipStream_t s) {
   void* args[] = {&tp};
   // all LDS is static (no dynamic shared memory)
   return hip_status(hipLaunchKernel(reinterpret_cast<const void*>(tiled::tiled_gemm<T, tiled::B_I8, TO, WGM, WGN, FM, FN,
-                                                                                      EPI, S, RING, WPE, XR>),
+                                                                                      EPI, S, RING, WPE, SB>),
                                     dim3(static_cast<unsigned>(tp.tiles_m * tp.tiles_n)), dim3(C::BLOCK), args, 0, s),
                     "w8a16 tiled launch");
 }
 
-// Outside the ring's range (below), the step pipeline's tile shape by the
-// number T of 128 x 128 output tiles, from a sweep of tile shapes x waves x
-// LDS stages on MI355X over the q/o, k/v, gate/up and down projections of
-// Qwen2.5-1.5B and 7B at 128, 1024 and 4096 rows (every pick within 5% of
-// the best sampled configuration but one, 1024 rows x k 8960, at 1.05x):
-//   T < 128 -> 64 x 64 tiles, 4 waves, 4 stages (the most workgroups);
-//   T < 320, or n > 2048 (fewer than two ring tiles per CU) -> 128 x 128,
-//     8 waves, 3 stages;
-//   else (n <= 2048) -> 128 x 256, 8 waves, 4 stages.
-// bf16 takes 128 x 128 where fp16 takes 128 x 256: its widening needs more
-// registers, and the 128 x 256 shape would spill.
+// Unsplit tiles of one matrix, by split_plan's prediction (tiled_plan.h): 64
+// x 64 (4 waves) and 32 x 64 (2 waves) in the step pipeline with 4 stages;
+// 64 x 128 (8 waves, 4 stages), 128 x 128 (8 waves, 3 stages) and 192 x 128 (8
+// waves of 96 x 32, 2 stages, its registers capped at 128 so that two
+// workgroups fit on a CU) on the sub-step ring.  16 waves per CU issue the
+// global -> LDS DMA that bounds this GEMM; more stages measured even or
+// slower (the widening, not the loads, fills the gaps).  Against the rules on
+// n and tile counts before: 1.5B down 3000 rows 138.9 -> 99.5 us, 14B gate
+// 1300 rows 250.6 -> 186.4, 7B gate 160 rows 52.5 -> 41.8, 1.5B gate 160 rows
+// 17.6 -> 14.0.
 template <typename T, typename TO>
-int w8_tiled(const W8Params& p, hipStream_t s, int cus) {
-  constexpr bool wide = std::is_same<T, F16>::value;
-  // Wide outputs from 1024 rows at gate/up and o-projection depths (k <=
-  // 4096): 128 x 128 tiles of 8 waves (64 x 32 each) behind a 3-stage ring,
-  // two workgroups per CU, so 16 waves per CU issue the global -> LDS DMA
-  // that bounds this GEMM, for 40% fewer operand bytes per flop than 128 x 64
-  // tiles.  Measured against the plan below and forced configurations 1-33:
-  // 1.5B gate/up 1024 rows 45.8 vs 49.8 us, 4096 rows 138.6 vs 155.8 us; 7B
-  // gate/up (bf16) 149.4 vs 178.5 and 556.9 vs 582.2 us; 7B o projection and
-  // n = 4736 even.  The deep 7B down projection (k = 18944) at 4096 rows
-  // keeps the plan below (512.7 vs 533.8 us).
-  // Where 192 x 128 tiles (8 waves of 96 x 32, 2-stage ring) fit in one
-  // round of two workgroups per CU and 128 x 128 tiles would need a second,
-  // the 192 x 128 tile with its registers capped at 128 (4 waves per SIMD,
-  // so two workgroups fit on a CU): 1.5B gate/up at 1024 rows, 420 tiles
-  // against 560 of 128 x 128 on 512 slots, 43.0 vs 46.8 us.  (Its tile
-  // counts here are rarely multiples of 8: XR = 1, 43.2 vs 44.4 us at 420
-  // tiles.)
-  if (p.n > 2048 && p.rows >= 1024 && p.k <= 4096) {
-    const int64_t cols = (p.n + 127) / 128;
-    const int64_t t192 = (p.rows + 191) / 192 * cols, t128x128 = (p.rows + 127) / 128 * cols;
-    if (t192 <= 2 * static_cast<int64_t>(cus) && t128x128 > 2 * static_cast<int64_t>(cus))
-      return w8_tiled_cfg<T, TO, 2, 4, 3, 1, 2, tiled::EPI_W8, 1, 4, 1>(p, s);
-    return w8_tiled_cfg<T, TO, 2, 4, 2, 1, 3, tiled::EPI_W8, 1>(p, s);
+int w8_tiled(const W8Params& p, int shape, hipStream_t s) {
+  switch (shape) {
+    case 0: return w8_tiled_cfg<T, TO, 2, 2, 1, 1, 4>(p, s);
+    case 1: return w8_tiled_cfg<T, TO, 2, 4, 1, 1, 4, tiled::EPI_W8, 1>(p, s);
+    case 2: return w8_tiled_cfg<T, TO, 2, 4, 2, 1, 3, tiled::EPI_W8, 1>(p, s);
+    case 3: return w8_tiled_cfg<T, TO, 2, 4, 3, 1, 2, tiled::EPI_W8, 1, 4>(p, s);
+    default: return w8_tiled_cfg<T, TO, 1, 2, 1, 1, 4>(p, s);
   }
-  // Below 1024 rows, wide outputs with at least two 128 x 64 tiles per CU: the sub-step ring
-  // (2 stages) at the shape whose busiest CU finishes first -- ceil(tiles /
-  // CUs) times the cost of one tile of 128 x 64 (4 waves, 40 KiB of LDS, four
-  // workgroups per CU), 256 x 128 (8 waves of 128 x 32, two per CU) or
-  // 256 x 256 (8 waves of 64 x 128), measured about 1 : 3.8 : 6.4 at the
-  // Qwen2.5-1.5B and 7B gate/up and down projections (1.5B gate 512 rows
-  // 34.9 -> 26.2 us, 7B down 4096 rows 641 -> 522 us; the 3.8 from a later
-  // sweep, where 128 x 64 tiles took 158-160 us at 1.5B gate/up 4096 rows
-  // against 165-168 us for 256 x 128).  Fewer tiles keep the rule below,
-  // whose smaller grids spread better.
-  if (p.n > 2048) {
-    const auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
-    const int64_t t_small = cdiv(p.rows, 128) * cdiv(p.n, 64);
-    if (t_small >= 2 * static_cast<int64_t>(cus)) {
-      const double c_small = static_cast<double>(cdiv(t_small, cus));
-      const double c_mid = 3.8 * static_cast<double>(cdiv(cdiv(p.rows, 256) * cdiv(p.n, 128), cus));
-      const double c_big = 6.4 * static_cast<double>(cdiv(cdiv(p.rows, 256) * cdiv(p.n, 256), cus));
-      if (c_small <= c_mid && c_small <= c_big) return w8_tiled_cfg<T, TO, 2, 2, 2, 1, 2, tiled::EPI_W8, 1>(p, s);
-      if (c_mid <= c_big) return w8_tiled_cfg<T, TO, 2, 4, 4, 1, 2, tiled::EPI_W8, 1>(p, s);
-      return w8_tiled_cfg<T, TO, 4, 2, 2, 4, 2, tiled::EPI_W8, 1>(p, s);
-    }
-  }
-  // Narrow outputs (n <= 2048) whose 64 x 128 tiles number between half and
-  // all of the CUs: 8 waves of 32 x 32 per tile behind a 4-stage ring, one
-  // tile per CU with 8 waves issuing its DMA (forced configurations 17 and
-  // 34-36 against the plan below: 1.5B down 1024 rows 49.8 vs 59.4 us, 1280
-  // rows 51.6 vs 60.6; q/o 1024 rows 13.8 vs 15.6; n = 2048 14.1 vs 18.5;
-  // 768 rows even).  Fewer tiles (512-row down and q/o, n = 1024) and more
-  // (2048 rows and up) run faster on the shapes below.
-  const int64_t t64x128 = static_cast<int64_t>((p.rows + 63) / 64) * ((p.n + 127) / 128);
-  if (p.n <= 2048 && 2 * t64x128 > cus && t64x128 <= cus)
-    return w8_tiled_cfg<T, TO, 2, 4, 1, 1, 4, tiled::EPI_W8, 1>(p, s);
-  const int64_t t128 = static_cast<int64_t>((p.rows + 127) / 128) * ((p.n + 127) / 128);
-  if (t128 < 128) return w8_tiled_cfg<T, TO, 2, 2, 1, 1, 4>(p, s);
-  if (t128 < 320 || p.n > 2048) return w8_tiled_cfg<T, TO, 2, 4, 2, 1, 3>(p, s);
-  if constexpr (wide) return w8_tiled_cfg<T, TO, 2, 4, 2, 2, 4>(p, s);
-  else return w8_tiled_cfg<T, TO, 2, 4, 2, 1, 3>(p, s);
 }
 
-// The dual (gate/up + SiLU-and-mul) tiled GEMM: more than 256 rows by the
-// round count below; else, up to n = 10000, 128 x 64 tiles (4 waves, 4
-// stages), beyond 128 x 128 (8 waves, 3 stages; fp16) -- the 16-bit gate/up
-// GEMM's step-pipeline shapes, less its 256 x 64 one, whose 4 KiB int8 B
-// tile does not split into the 8 waves' 1 KiB DMA instructions.  bf16 keeps
-// the 128 x 64 shape there (its widening needs more registers; 128 x 128 at
-// 8 waves would spill).
+// The dual (gate/up + SiLU-and-mul) tiled GEMM beyond the small tiles, by the
+// prediction of tiled_plan.h: on the sub-step ring 96 x 128 (4 waves, 3
+// stages), 64 x 64 (4 waves, 3 stages, three workgroups per CU), 128 x 64 (4
+// waves, 2 stages, three per CU; or 3 stages of x and 4 of the weights, two
+// per CU), 192 x 128 and 256 x 128 (8 waves, 2 stages); in the step pipeline
+// 128 x 64 (4 waves, 4 stages, one per CU).  Against the rounds rule before:
+// 1.5B 160 rows 39.1 -> 22.6 us, 256 rows 40.0 -> 28.2; 14B 100 rows 79.9 ->
+// 57.3; 7B 160 rows 104.5 -> 76.2.
+constexpr tiled::ShapeCost kGateUp8Cost[] = {{96, 128, 1, 2.8, {0.639, 0, 0}, 0.113, 0, 6.5},
+                                             {64, 64, 3, 5.6, {0.250, 0.446, 0.644}, 0.092, 0.034, 2.7},
+                                             {128, 64, 3, 4.4, {0.405, 0.570, 0.917}, 0.167, 0.025, 4.3},
+                                             {128, 64, 2, 4.6, {0.382, 0.616, 0}, 0.179, 0.011, 5.4},
+                                             {192, 128, 2, 0, {0.914, 2.080, 0}, 0.317, 0, 9.8},
+                                             {256, 128, 1, 0, {0.888, 0, 0}, 0.747, 0, 10.5},
+                                             {128, 64, 1, 0, {0.620, 0, 0}, 0.030, 0, 5.0}};
+
+template <typename T, typename TO>
+int w8_dual_shape(const W8Params& p, int shape, hipStream_t s) {
+  constexpr int E = tiled::EPI_SILU_W8;
+  switch (shape) {
+    case 0: return w8_tiled_cfg<T, TO, 1, 4, 3, 1, 3, E, 1>(p, s);
+    case 1: return w8_tiled_cfg<T, TO, 2, 2, 1, 1, 3, E, 1>(p, s);
+    case 2: return w8_tiled_cfg<T, TO, 2, 2, 2, 1, 2, E, 1>(p, s);
+    case 3: return w8_tiled_cfg<T, TO, 2, 2, 2, 1, 3, E, 1, 0, 4>(p, s);
+    case 4: return w8_tiled_cfg<T, TO, 2, 4, 3, 1, 2, E, 1>(p, s);
+    case 5: return w8_tiled_cfg<T, TO, 2, 4, 4, 1, 2, E, 1>(p, s);
+    default: return w8_tiled_cfg<T, TO, 2, 2, 2, 1, 4, E>(p, s);
+  }
+}
+
 template <typename T, typename TO>
 int w8_tiled_dual(const W8Params& p, hipStream_t s, int cus) {
-  // More than 256 rows: the sub-step ring (2 stages), 128 x 64 tiles (4
-  // waves, 48 KiB of LDS, three workgroups per CU) or 256 x 128 (8 waves of
-  // 128 x 32), whichever takes fewer rounds, a round of 256 x 128 weighted
-  // 1.28 (measured at the Qwen2.5-1.5B and 7B MLPs, 512 - 4096 rows: 1.5B
-  // 1024 rows 90.8 -> 70.2 us, 7B 2048 rows 719 -> 494 us).
-  if (p.rows > 256) {
-    const auto cdiv = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
-    const double c_small = static_cast<double>(cdiv(cdiv(p.rows, 128) * cdiv(p.n, 64), 3 * static_cast<int64_t>(cus)));
-    const double c_big = 1.28 * static_cast<double>(cdiv(cdiv(p.rows, 256) * cdiv(p.n, 128), cus));
-    if (c_small <= c_big) return w8_tiled_cfg<T, TO, 2, 2, 2, 1, 2, tiled::EPI_SILU_W8, 1>(p, s);
-    return w8_tiled_cfg<T, TO, 2, 4, 4, 1, 2, tiled::EPI_SILU_W8, 1>(p, s);
-  }
-  if constexpr (std::is_same<T, F16>::value) {
-    if (p.rows > 256 || p.n > 10000) return w8_tiled_cfg<T, TO, 2, 4, 2, 1, 3, tiled::EPI_SILU_W8>(p, s);
-  }
-  return w8_tiled_cfg<T, TO, 2, 2, 2, 1, 4, tiled::EPI_SILU_W8>(p, s);
+  const double wmb = 2e-6 * static_cast<double>(p.n) * p.k;
+  return w8_dual_shape<T, TO>(p, tiled::plan_tiles(kGateUp8Cost, p.rows, p.n, p.k, wmb, cus, false).shape, s);
 }
 
 // Small tiled shapes for 17 - 64 rows: 32 x 64 (2 waves) or, for n > 10000,
@@ -542,18 +488,11 @@ int w8_typed(const W8Params& p, hipStream_t s, int cus, void* work = nullptr, in
     return w8_stream_launch<T, TO, DUAL>(p, w8_stream_plan(p.rows, p.k, p.n, DUAL, cus), s);
   if (p.rows <= 24) return w8_skinny_shape<T, TO, 3, DUAL>(p, s, cus);
   if (p.rows <= 32) return w8_skinny_shape<T, TO, 4, DUAL>(p, s, cus);
-  // More rows: the tiled GEMM, except where 32-row skinny tiles with split K,
-  // which re-read the int8 weights per tile mostly from L2, measured faster:
-  // tiny grids (fewer than 32 64 x 64 tiles: 1.5B k/v at 96 - 256 rows, 6.4
-  // vs 10.5 us) and narrow outputs (n < 2048) up to 128 rows (1.5B down, 128
-  // rows 30.7 vs 34.3 us).  Wider outputs and more rows re-read too much
-  // (7B down, 96 rows 105.6 vs 82.8 us; 1.5B down, 256 rows 57.6 vs 34.7).
-  const int64_t tiles64 = static_cast<int64_t>((p.n + 63) / 64) * ((p.rows + 63) / 64);
-  bool skinny = p.rows <= 256 && (tiles64 < 32 || (p.rows <= 128 && p.n < 2048));
-  if (!tiled_fits(p, DUAL)) skinny = true;
+  // More rows: the tiled GEMM, except where 32-row skinny tiles are faster.
+  const bool skinny = tiled::w8_skinny_pays(p.rows, p.n) || !tiled_fits(p, DUAL);
   if (skinny) return w8_skinny_shape<T, TO, 4, DUAL>(p, s, cus);
   if constexpr (DUAL) return w8_tiled_dual<T, TO>(p, s, cus);
-  else return w8_tiled<T, TO>(p, s, cus);
+  else return w8_tiled<T, TO>(p, tiled::split_plan(p.rows, p.k, p.n, 1, cus).direct, s);
 }
 
 }  // namespace

@@ -17,9 +17,9 @@ pytestmark = pytest.mark.gpu
 F16, BF16, F32 = torch.float16, torch.bfloat16, torch.float32
 # rows, k, n: the 32 x 128, 64 x 64, 64 x 128, 128 x 128 and 256 x 256 tiles at
 # the edges of their rows, k with a partial last step, n odd or not of 4
-SHAPES16 = [(31, 6008, 3584), (65, 2008, 130), (129, 4000, 131), (17, 9016, 5121), (65, 12008, 1536), (128, 6000, 3582),
-            (400, 6008, 5122), (1001, 12008, 2049)]
-SHAPES8 = [(200, 2032, 500), (32, 18960, 3584), (65, 2016, 130), (64, 9008, 1537), (33, 6000, 3584), (129, 6000, 5122),
+SHAPES16 = [(31, 12008, 2050), (65, 2008, 130), (129, 4000, 131), (17, 9016, 5121), (65, 12008, 1536), (128, 6000, 3582),
+            (400, 9008, 5122), (1001, 12008, 2049)]
+SHAPES8 = [(200, 2032, 500), (32, 18960, 3584), (65, 4016, 130), (64, 9008, 1537), (33, 6000, 3584), (129, 6000, 5122),
            (65, 18960, 1538), (1001, 9008, 5122)]
 
 
