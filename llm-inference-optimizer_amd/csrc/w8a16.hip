@@ -382,7 +382,7 @@ int w8_tiled(const W8Params& p, int shape, hipStream_t s) {
 // The dual (gate/up + SiLU-and-mul) tiled GEMM beyond the small tiles, by the
 // prediction of tiled_plan.h: on the sub-step ring 96 x 128 (4 waves, 3
 // stages), 64 x 64 (4 waves, 3 stages, three workgroups per CU), 128 x 64 (4
-// waves, 2 stages, three per CU; or 3 stages of x and 4 of the weights, two
+// waves, 2 stages, its registers capped so that three fit per CU; or 3 stages of x and 4 of the weights, two
 // per CU), 192 x 128 and 256 x 128 (8 waves, 2 stages); in the step pipeline
 // 128 x 64 (4 waves, 4 stages, one per CU).  Against the rounds rule before:
 // 1.5B 160 rows 39.1 -> 22.6 us, 256 rows 40.0 -> 28.2; 14B 100 rows 79.9 ->
@@ -401,7 +401,7 @@ int w8_dual_shape(const W8Params& p, int shape, hipStream_t s) {
   switch (shape) {
     case 0: return w8_tiled_cfg<T, TO, 1, 4, 3, 1, 3, E, 1>(p, s);
     case 1: return w8_tiled_cfg<T, TO, 2, 2, 1, 1, 3, E, 1>(p, s);
-    case 2: return w8_tiled_cfg<T, TO, 2, 2, 2, 1, 2, E, 1>(p, s);
+    case 2: return w8_tiled_cfg<T, TO, 2, 2, 2, 1, 2, E, 1, 3>(p, s);
     case 3: return w8_tiled_cfg<T, TO, 2, 2, 2, 1, 3, E, 1, 0, 4>(p, s);
     case 4: return w8_tiled_cfg<T, TO, 2, 4, 3, 1, 2, E, 1>(p, s);
     case 5: return w8_tiled_cfg<T, TO, 2, 4, 4, 1, 2, E, 1>(p, s);
