@@ -691,6 +691,8 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
   int el = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
   asm volatile("" : "+v"(el));
   const int er = el & 31, eh = el >> 5;
+  // 16-bit rows of whole 8-byte quads only: four columns a lane, straight from the accumulators
+  const bool quads = os % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0;
   wait_vmcnt<0>();  // no copy into the stage is in flight, and every wave is past its last read
   lds_barrier();
   // scalar copies: the per-lane use of the originals would pull the buffer
@@ -773,10 +775,19 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
           if (ml < nrows_x) {
 #pragma unroll
             for (int g = 0; g < GP; ++g) {
+              const int nl = nj + 8 * (gp + g) + 4 * eh;
+              const int64_t o = static_cast<int64_t>(m0 + ml) * os + n0 + nl;
+              if (ES == 2 && quads && nl + 4 <= nrows_b) {
+                if constexpr (ES == 2) {
+                  const f32x2 lo = {v[g][0], v[g][1]}, hi = {v[g][2], v[g][3]};
+                  *reinterpret_cast<u32x2*>(static_cast<typename TO::bits*>(out) + o) =
+                      u32x2{narrow2<TO>(lo), narrow2<TO>(hi)};
+                }
+                continue;
+              }
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
-                const int nl = nj + 8 * (gp + g) + 4 * eh + e;
-                if (nl < nrows_b) store_elem<TO>(out, static_cast<int64_t>(m0 + ml) * os + n0 + nl, v[g][e]);
+                if (nl + e < nrows_b) store_elem<TO>(out, o + e, v[g][e]);
               }
             }
           }

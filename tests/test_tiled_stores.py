@@ -1,7 +1,7 @@
 """The tiled kernels' output stores (csrc/tiled_gemm.h): 64-byte row segments
 through LDS where the output's row stride and address allow 16-byte stores,
-single elements otherwise, ragged last segments and rows in both.  The same
-call into an aligned, a wider and a misaligned output through the C ABI gives
+8-byte stores or single elements otherwise, ragged last segments and rows in
+each.  The same call into outputs of those four kinds through the C ABI gives
 the same values (equal bits: one kernel, one summation order), and nothing
 outside the output's columns is written."""
 import importlib
@@ -47,7 +47,7 @@ def test_output_layouts(pkg, cuda, rows, n, out_dt, int8):
     odt = dt if out_dt == "half" else F32
     wide = (n + 23) // 8 * 8  # a row stride of whole 16-byte packets, at least 16 columns of guard
     got = []
-    for os, off in ((wide, 0), (wide, 1), (n + 17, 0)):
+    for os, off in ((wide, 0), (wide, 1), (n + 17, 0), (wide + 4, 0)):
         buf = torch.full((rows * os + 64,), 77.0, device=cuda, dtype=odt)
         view = buf[off:off + rows * os].view(rows, os)
         assert _call(lib, int8, x, w, scale, bias, view, os, n) == 0
@@ -60,4 +60,4 @@ def test_output_layouts(pkg, cuda, rows, n, out_dt, int8):
     # fp32 sums of k terms and two more roundings, then one rounding to 16 bits
     eps = 2.0 ** -24 * (k + 4) + (0 if odt == F32 else 2.0 ** (-11 if dt == F16 else -8))
     assert float(((got[0].double() - exact).abs() - eps * mag).max()) <= 0
-    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
+    assert all(torch.equal(got[0], other) for other in got[1:])
