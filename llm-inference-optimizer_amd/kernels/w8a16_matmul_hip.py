@@ -6,7 +6,9 @@ output dtype and shapes of the reference's launcher
 replaced by hand-written HIP kernels behind the C ABI
 ``mi355_w8a16_linear_fwd``: a weight-streaming MFMA kernel for decode batches
 (<= 16 rows; up to 48 -- 64 for matrices of at most 8 MB -- where the
-small tiles do not pay), an LDS-tiled MFMA GEMM for larger ones.  Arithmetic as there:
+small tiles do not pay), an LDS-tiled MFMA GEMM for larger ones, split over K
+(from 17 rows) where the output alone would not fill the chip.  Arithmetic as
+there:
 ``out = (sum_k x * w_q) * scale + bias`` with the integer dot product in fp32,
 the scale applied once, one rounding to x's dtype.
 
