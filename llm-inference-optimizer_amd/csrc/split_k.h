@@ -154,8 +154,11 @@ inline SplitPlan split_plan(uint32_t rows, uint32_t k, uint32_t n, int wb, uint3
   for (int t = 0; t < SPLIT_TILES; ++t) {
     const double fixed = sc[t].c0 + sc[t].weight * wmb;
     if (fixed >= limit) continue;
-    const uint32_t tiles = plan_cdiv(rows, static_cast<uint32_t>(sc[t].bm)) * plan_cdiv(n, static_cast<uint32_t>(sc[t].bn));
-    if (2 * tiles > cus) continue;
+    // 64 bits: the size query takes any rows and n below 2^31, beyond what a launch may hold
+    const uint64_t all = static_cast<uint64_t>(plan_cdiv(rows, static_cast<uint32_t>(sc[t].bm))) *
+                         plan_cdiv(n, static_cast<uint32_t>(sc[t].bn));
+    if (2 * all > cus) continue;
+    const uint32_t tiles = static_cast<uint32_t>(all);
     uint32_t s = cus / tiles;
     if (s > 32) s = 32;
     if (s > steps / 4) s = steps / 4;

@@ -2,8 +2,11 @@
 the probe library; no GPU call): over row counts, widths and depths of any
 alignment, a plan that splits gives every K range work, starts no more
 workgroups than the CUs, and wants a workspace of exactly its fp32 sums,
-bounded by one largest tile per CU; decode rows and wide outputs never split."""
+bounded by one largest tile per CU; decode rows and wide outputs never split;
+sizes beyond any launch are answered, not divided by."""
 import ctypes
+import subprocess
+import sys
 from pathlib import Path
 
 import pytest
@@ -47,3 +50,26 @@ def test_split_plan_is_launchable(plan, wb, cus):
                 assert nbytes == 4 * splits * rows * n <= 4 * cus * 256 * 256
     if cus == 256:
         assert tiles_seen == set(range(5)), tiles_seen
+
+
+@pytest.mark.parametrize("wb", [1, 2])
+def test_sizes_beyond_a_launch_want_no_workspace(wb):
+    # Tile counts that are multiples of 2^32, or wrap to a few: the size query
+    # takes any rows, k, n below 2^31.  In a child process, which a division
+    # by zero would end.
+    if not PROBE.exists():
+        pytest.skip("probe library not built")
+    code = f"""
+import ctypes
+f = ctypes.CDLL({str(PROBE)!r}).mi355_probe_split_plan
+f.argtypes, f.restype = [ctypes.c_longlong] * 3 + [ctypes.c_int] * 2 + [ctypes.c_void_p], ctypes.c_longlong
+out = (ctypes.c_int * 4)()
+near = [v for e in range(8, 32) for v in (2 ** e - 1, 2 ** e, 2 ** e + 1) if v < 2 ** 31]
+for rows in near:
+    for n in near:
+        if rows * n > 2 ** 34:
+            for k in (64, 4096, 2 ** 31 - 1):
+                assert f(rows, k, n, {wb}, 256, out) == 0 and out[0] < 0, (rows, k, n)
+"""
+    res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
+    assert res.returncode == 0, (res.returncode, res.stderr)
