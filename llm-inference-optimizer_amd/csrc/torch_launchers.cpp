@@ -145,11 +145,26 @@ std::vector<int64_t> with_last(at::IntArrayRef s, int64_t last) {
 
 void* ptr(const at::Tensor& t) { return t.data_ptr(); }
 
+// Whether the split-K kernels take these operands (the alignment that the
+// linears' launchers ask of everything but their generic kernels): row starts
+// on 16 bytes, whole 16-byte packets per row.
+bool packets(const at::Tensor& x, int64_t xs, const at::Tensor& w, int64_t ws, int64_t k) {
+  const int64_t xe = x.element_size(), we = w.element_size();
+  return xs * xe % 16 == 0 && ws * we % 16 == 0 && k * we % 16 == 0 &&
+         (reinterpret_cast<uintptr_t>(ptr(x)) | reinterpret_cast<uintptr_t>(ptr(w))) % 16 == 0;
+}
+
 // A call's scratch memory: `bytes` from torch's allocator on the current
 // stream (the launch stream, so its reuse is ordered after the call's kernels;
-// a captured graph keeps it in its pool), or an undefined tensor for 0.
+// a captured graph keeps it in its pool).  Undefined for 0 bytes, and where
+// the memory is not to be had: the call then runs the unsplit kernels.
 at::Tensor workspace(int64_t bytes, const at::Tensor& like) {
-  return bytes > 0 ? at::empty({bytes}, like.options().dtype(at::kByte)) : at::Tensor();
+  if (bytes <= 0) return {};
+  try {
+    return at::empty({bytes}, like.options().dtype(at::kByte));
+  } catch (const c10::OutOfMemoryError&) {
+    return {};
+  }
 }
 
 // ------------------------------------------------------------------ RMSNorm
@@ -306,7 +321,7 @@ at::Tensor linear16(const at::Tensor& x, const at::Tensor& weight, const c10::op
     const int64_t xs = M > 1 ? x2.stride(0) : K;
     const int64_t ws = N > 1 ? w.stride(0) : K;
     Launch l(dev);
-    const at::Tensor work = workspace(mi355_linear16_workspace(M, K, N), x);
+    const at::Tensor work = workspace(packets(x2, xs, w, ws, K) ? mi355_linear16_workspace(M, K, N) : 0, x);
     check("mi355_linear16_fwd",
           mi355_linear16_ws_fwd(ptr(x2), ptr(w), has_bias ? ptr(b) : nullptr, ptr(out), M, K, N, xs, ws, N,
                                 code_of(x.scalar_type()), has_bias ? code_of(b.scalar_type()) : 0, code_of(odt),
@@ -348,7 +363,7 @@ at::Tensor w8a16_linear(const at::Tensor& x, const at::Tensor& w_q, const at::Te
     const int64_t xs = M > 1 ? x2.stride(0) : K;
     const int64_t ws = N > 1 ? q.stride(0) : K;
     Launch l(dev);
-    const at::Tensor work = workspace(mi355_w8a16_linear_workspace(M, K, N), x);
+    const at::Tensor work = workspace(packets(x2, xs, q, ws, K) ? mi355_w8a16_linear_workspace(M, K, N) : 0, x);
     check("mi355_w8a16_linear_fwd",
           mi355_w8a16_linear_ws_fwd(ptr(x2), ptr(q), ptr(s), has_bias ? ptr(b) : nullptr, ptr(out), M, K, N, xs, ws, N,
                                     code_of(x.scalar_type()), code_of(s.scalar_type()),

@@ -106,3 +106,61 @@ def test_split_against_unsplit_and_strided_and_graph(pkg, cuda, lib, int8):
         graph.replay()
         assert torch.equal(out, want)
         assert torch.equal(call(x, w), want)
+
+
+def _linear(pkg, cuda, int8, rows, k, n):
+    x, w, s, _, _, _ = _case((rows, k, n), F16, cuda, int8, False)
+    return x, w, s, (lambda: pkg.w8a16_linear(x, w, s)) if int8 else (lambda: pkg.linear16(x, w))
+
+
+@pytest.mark.parametrize("int8", [False, True])
+@pytest.mark.parametrize("rows,k,n,offset", [(200, 4001, 500, 0), (200, 4008, 500, 1)])
+def test_no_workspace_where_split_k_cannot_run(pkg, cuda, int8, rows, k, n, offset):
+    """Rows that are no whole 16-byte packets run the generic kernel: such a
+    call allocates its output and nothing else."""
+    x = torch.randn(rows * k + offset, generator=gen(3)).to(F16).to(cuda)[offset:].view(rows, k)
+    if int8:
+        w, s = torch.randint(-127, 128, (n, k), device=cuda, dtype=torch.int8), torch.rand(n, device=cuda)
+        call = lambda: pkg.w8a16_linear(x, w, s)
+    else:
+        w = torch.randn(n, k, generator=gen(4)).to(F16).to(cuda)
+        call = lambda: pkg.linear16(x, w)
+    call()
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    out = call()
+    assert torch.cuda.max_memory_allocated() - before <= out.numel() * 2 + 512
+
+
+@pytest.mark.parametrize("int8", [False, True])
+def test_without_memory_for_the_workspace(pkg, cuda, lib, int8):
+    """A call whose output fits but whose workspace does not runs the unsplit
+    kernels, as one through the C ABI without a workspace does."""
+    rows, k, n = 700, 18944, 3584
+    torch.cuda.empty_cache()
+    x, w, s, call = _linear(pkg, cuda, int8, rows, k, n)
+    torch.cuda.empty_cache()  # every tensor of the test in a segment of its own
+    want = torch.empty(rows, n, dtype=F16, device=cuda)
+    stream = torch.cuda.current_stream().cuda_stream
+    if int8:
+        nbytes = lib.load().mi355_w8a16_linear_workspace(rows, k, n)
+        lib.w8a16_linear_fwd(x.data_ptr(), w.data_ptr(), s.data_ptr(), None, want.data_ptr(), rows, k, n, k, k, n,
+                             lib.F16, lib.F32, 0, lib.F16, stream)
+    else:
+        nbytes = lib.load().mi355_linear16_workspace(rows, k, n)
+        lib.linear16_fwd(x.data_ptr(), w.data_ptr(), None, want.data_ptr(), rows, k, n, k, k, n, lib.F16, 0, lib.F16,
+                         stream)
+    assert nbytes > 20 << 20, "must not fit the segment of the cached block below"
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.empty(rows, n, dtype=F16, device=cuda)  # freed: a cached block for the output
+    try:
+        torch.cuda.set_per_process_memory_fraction(
+            torch.cuda.memory_reserved() / torch.cuda.get_device_properties(cuda).total_memory)
+        with pytest.raises(torch.OutOfMemoryError):
+            torch.empty(nbytes, dtype=torch.uint8, device=cuda)
+        got = call()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(got, want)
