@@ -7,6 +7,7 @@
 #include <cstdarg>
 #include <cstdio>
 
+#include "../quantize_plan.h"
 #include "../split_k.h"
 #include "../w8a16_stream.h"
 
@@ -267,4 +268,17 @@ extern "C" __attribute__((visibility("default"))) long long mi355_probe_split_pl
   out4[2] = sp.tile < 0 ? 0 : mi355::tiled::kSplitCost16[sp.tile].bm;
   out4[3] = sp.tile < 0 ? 0 : mi355::tiled::kSplitCost16[sp.tile].bn;
   return mi355::tiled::split_bytes(sp, rows, n);
+}
+
+// The quantiser's launch (quant_plan) of n rows of `packets` 16-byte packets:
+// out4 = {packets a lane (0: generic), workgroup per row, threads, 0}; returns
+// the workgroups.
+extern "C" __attribute__((visibility("default"))) long long mi355_probe_quant_plan(long long n, long long packets,
+                                                                                    int* out4) {
+  const mi355::QuantPlan p = mi355::quant_plan(n, packets);
+  out4[0] = p.vpl;
+  out4[1] = p.block ? 1 : 0;
+  out4[2] = p.threads;
+  out4[3] = 0;
+  return p.grid;
 }

@@ -27,6 +27,7 @@
 // kernel before (one wave per row, 2-byte loads, the row read twice, a
 // division per weight) 124.8 us.
 #include "common.h"
+#include "quantize_plan.h"
 
 namespace mi355 {
 namespace {
@@ -216,34 +217,29 @@ int launch_quant(K kernel, int64_t grid, int block, const QuantArgs& a, hipStrea
 }
 
 // Packets need whole ones per row, 16-byte aligned weight rows and code rows
-// aligned to a packet's codes; a row of more than 16 waves x 8 packets a lane
-// takes the generic kernel, as does a grid past 2^31 workgroups.
+// aligned to a packet's codes.
 template <typename TW>
 int quant_typed(const QuantArgs& a, hipStream_t s) {
   constexpr int W = pack_width<TW>::value;
   const int64_t eb = sizeof(typename TW::bits);
   const bool vec = a.k % W == 0 && aligned16(a.w) && a.ws * eb % 16 == 0 &&
                    reinterpret_cast<uintptr_t>(a.q) % W == 0 && a.qs % W == 0;
-  const int64_t rows4 = (a.n + 3) / 4;
-  const int nvec = a.k / W, vpl = (nvec + 63) / 64;
-  if (!vec || vpl > 16 * 8 || (vpl > 8 && a.n > 0x7fffffff))
-    return launch_quant(quantize_int8_generic<TW>, rows4, 256, a, s);
-  switch (vpl) {
-    case 1: return launch_quant(quantize_int8_rows<TW, 1, false>, rows4, 256, a, s);
-    case 2: return launch_quant(quantize_int8_rows<TW, 2, false>, rows4, 256, a, s);
-    case 3: return launch_quant(quantize_int8_rows<TW, 3, false>, rows4, 256, a, s);
-    case 4: return launch_quant(quantize_int8_rows<TW, 4, false>, rows4, 256, a, s);
-    case 5: return launch_quant(quantize_int8_rows<TW, 5, false>, rows4, 256, a, s);
-    case 6: return launch_quant(quantize_int8_rows<TW, 6, false>, rows4, 256, a, s);
-    case 7: return launch_quant(quantize_int8_rows<TW, 7, false>, rows4, 256, a, s);
-    case 8: return launch_quant(quantize_int8_rows<TW, 8, false>, rows4, 256, a, s);
-    default: break;
+  const QuantPlan p = quant_plan(a.n, vec ? a.k / W : 0);
+  if (p.block) {
+    if (p.vpl == 4) return launch_quant(quantize_int8_rows<TW, 4, true>, p.grid, p.threads, a, s);
+    return launch_quant(quantize_int8_rows<TW, 8, true>, p.grid, p.threads, a, s);
   }
-  if (vpl <= 16 * 4) {
-    const int waves = (vpl + 3) / 4;
-    return launch_quant(quantize_int8_rows<TW, 4, true>, a.n, 64 * waves, a, s);
+  switch (p.vpl) {
+    case 1: return launch_quant(quantize_int8_rows<TW, 1, false>, p.grid, p.threads, a, s);
+    case 2: return launch_quant(quantize_int8_rows<TW, 2, false>, p.grid, p.threads, a, s);
+    case 3: return launch_quant(quantize_int8_rows<TW, 3, false>, p.grid, p.threads, a, s);
+    case 4: return launch_quant(quantize_int8_rows<TW, 4, false>, p.grid, p.threads, a, s);
+    case 5: return launch_quant(quantize_int8_rows<TW, 5, false>, p.grid, p.threads, a, s);
+    case 6: return launch_quant(quantize_int8_rows<TW, 6, false>, p.grid, p.threads, a, s);
+    case 7: return launch_quant(quantize_int8_rows<TW, 7, false>, p.grid, p.threads, a, s);
+    case 8: return launch_quant(quantize_int8_rows<TW, 8, false>, p.grid, p.threads, a, s);
+    default: return launch_quant(quantize_int8_generic<TW>, p.grid, p.threads, a, s);
   }
-  return launch_quant(quantize_int8_rows<TW, 8, true>, a.n, 64 * ((vpl + 7) / 8), a, s);
 }
 
 }  // namespace
