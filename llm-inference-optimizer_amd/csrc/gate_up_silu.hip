@@ -279,13 +279,6 @@ int gate_up_tiled_cfg(const GateUpParams& p, hipStream_t s) {
 // 63.5 on 192 x 128).
 // Against the shapes and rounds rule before: 1.5B 389 rows 42.7 -> 32.9 us,
 // 7B 512 rows 164 -> 137, 0.5B 128 rows 11.2 -> 7.8, 14B 64 rows 90.6 -> 56.8.
-constexpr tiled::ShapeCost kGateUpCost[] = {{64, 64, 2, 1.7, {0.328, 0.551, 0}, 0.055, 0.101, 0},
-                                            {128, 64, 2, 3.6, {0.347, 0.715, 0}, 0.130, 0.038, 1.5},
-                                            {128, 128, 1, 1.6, {0.655, 0, 0}, 0.277, 0.035, 2.7},
-                                            {192, 128, 1, 1.3, {0.772, 0, 0}, 0.405, 0.007, 6.6},
-                                            {256, 128, 1, 1.4, {0.889, 0, 0}, 0.650, 0, 8.6},
-                                            {256, 64, 1, 0.1, {0.516, 0, 0}, 0.261, 0.068, 5.2}};
-
 template <typename T, typename TO>
 int gate_up_shape_launch(const GateUpParams& p, int shape, hipStream_t s) {
   switch (shape) {
@@ -313,7 +306,7 @@ int gate_up_tiled(const GateUpParams& p, hipStream_t s) {
   const int st = compute_units(&cus);
   if (st != MI355_OK) return st;
   const double wmb = 4e-6 * static_cast<double>(p.n_out) * p.k;
-  const tiled::TilePlan tp = tiled::plan_tiles(kGateUpCost, p.rows, p.n_out, p.k, wmb, cus, true);
+  const tiled::TilePlan tp = tiled::plan_tiles(tiled::kGateUpCost, p.rows, p.n_out, p.k, wmb, cus, true);
   if (tp.lead == 0) return gate_up_shape_launch<T, TO>(p, tp.shape, s);
   GateUpParams head = p, tail = p;
   head.n_out = tp.lead;

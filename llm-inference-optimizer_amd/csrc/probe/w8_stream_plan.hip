@@ -282,3 +282,28 @@ extern "C" __attribute__((visibility("default"))) long long mi355_probe_quant_pl
   out4[3] = 0;
   return p.grid;
 }
+
+// The unsplit tile plan (plan_tiles) over table 0: the 16-bit linear, 1: the
+// int8 linear, 2: the 16-bit gate/up, 3: the int8 gate/up of a [rows, k] x [n,
+// k] product on `cus` CUs: out9 = {shape, leading columns of a two-launch plan
+// (0: one launch), the rest's shape, then rows, columns and threads of the
+// first and of the second shape's workgroups}; returns the predicted us.
+extern "C" __attribute__((visibility("default"))) double mi355_probe_tile_plan(int table, long long rows, long long k,
+                                                                                long long n, int cus, int* out9) {
+  using namespace mi355::tiled;
+  const double nk = 1e-6 * static_cast<double>(n) * static_cast<double>(k);
+  auto run = [&](const auto& costs, double bytes, bool split) {
+    const TilePlan tp = plan_tiles(costs, static_cast<uint32_t>(rows), static_cast<uint32_t>(n),
+                                   static_cast<uint32_t>(k), bytes * nk, static_cast<uint32_t>(cus), split);
+    const ShapeCost &a = costs[tp.shape], &b = costs[tp.tail];
+    const int out[9] = {tp.shape, tp.lead, tp.tail, a.bm, a.bn, a.threads, b.bm, b.bn, b.threads};
+    for (int i = 0; i < 9; ++i) out9[i] = out[i];
+    return tp.cost;
+  };
+  switch (table) {
+    case 0: return run(kL16Cost, 2.0, false);
+    case 1: return run(kW8Cost, 1.0, false);
+    case 2: return run(kGateUpCost, 4.0, true);
+    default: return run(kGateUp8Cost, 2.0, false);
+  }
+}

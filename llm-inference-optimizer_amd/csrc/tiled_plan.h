@@ -24,17 +24,25 @@ namespace tiled {
 // `round` is a tile's first loads and its epilogue, which nothing overlaps
 // where a CU holds one workgroup.
 struct ShapeCost {
-  int bm, bn, occ;
+  int bm, bn, threads, occ;  // threads per workgroup
   double c0, step[3], load, weight, round;
 };
 
-// (32-bit: the launchers bound rows, n, k and rows * n / 4 below 2^31.  The
-// plan runs in every call; with 64-bit divisions it cost one about 0.6 us, as
-// here, with constant tile sizes, one plan takes 0.02 us.)
+// (32-bit divisions: the plan runs in every call; with 64-bit ones it cost a
+// call about 0.6 us, as here, with constant tile sizes, 0.02 us.)
 inline uint32_t plan_cdiv(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 
-__attribute__((always_inline)) inline double shape_time(const ShapeCost& s, uint32_t rows, uint32_t cols, uint32_t k, double wmb, uint32_t cus) {
-  const uint32_t tiles = plan_cdiv(rows, static_cast<uint32_t>(s.bm)) * plan_cdiv(cols, static_cast<uint32_t>(s.bn));
+// The time of a launch that holds 2^32 threads or more, which the runtime
+// refuses: 65 - 512 rows of 2^28 columns and more reach that with small tiles,
+// where larger ones (fewer threads per output element) still hold them.
+constexpr double kNoLaunch = 1e30;
+
+__attribute__((always_inline)) inline double shape_time(const ShapeCost& s, uint32_t rows, uint32_t cols, uint32_t k,
+                                                        double wmb, uint32_t cus) {
+  const uint64_t all = static_cast<uint64_t>(plan_cdiv(rows, static_cast<uint32_t>(s.bm))) *
+                       plan_cdiv(cols, static_cast<uint32_t>(s.bn));
+  if (all > 0xffffffffu / static_cast<uint32_t>(s.threads)) return kNoLaunch;
+  const uint32_t tiles = static_cast<uint32_t>(all);
   const uint32_t slots = cus * static_cast<uint32_t>(s.occ);
   const uint32_t full = tiles / slots, rest = tiles - full * slots;
   double per_step = full * s.step[s.occ - 1] + s.load * tiles / cus;
@@ -56,9 +64,9 @@ struct TilePlan {
 // the lead's tiles fill its rounds in order.)  wmb: MB of weights over all n
 // columns.
 template <int N>
-__attribute__((always_inline)) inline TilePlan plan_tiles(const ShapeCost (&table)[N], uint32_t rows, uint32_t n, uint32_t k, double wmb,
-                           uint32_t cus, bool split) {
-  TilePlan best{0, 0, 0, 1e30};
+__attribute__((always_inline)) inline TilePlan plan_tiles(const ShapeCost (&table)[N], uint32_t rows, uint32_t n,
+                                                          uint32_t k, double wmb, uint32_t cus, bool split) {
+  TilePlan best{0, 0, 0, kNoLaunch};
 #pragma unroll
   for (int i = 0; i < N; ++i) {  // unrolled: the table's tile sizes become constants
     const double c = shape_time(table[i], rows, n, k, wmb, cus);
@@ -87,20 +95,37 @@ __attribute__((always_inline)) inline TilePlan plan_tiles(const ShapeCost (&tabl
 
 // One int8 matrix (w8a16.hip): 64 x 64, 64 x 128, 128 x 128, 192 x 128 (capped
 // at 128 registers, two per CU) and 32 x 64.
-constexpr ShapeCost kW8Cost[] = {{64, 64, 3, 6.1, {0.181, 0.262, 0.400}, 0.060, 0.050, 0},
-                                 {64, 128, 2, 2.8, {0.250, 0.432, 0}, 0.101, 0.026, 3.4},
-                                 {128, 128, 2, 3.2, {0.288, 0.557, 0}, 0.216, 0.001, 5.0},
-                                 {192, 128, 2, 3.0, {0.429, 0.761, 0}, 0.322, 0, 6.5},
-                                 {32, 64, 3, 5.5, {0.177, 0.262, 0.282}, 0.022, 0.052, 0}};
+constexpr ShapeCost kW8Cost[] = {{64, 64, 256, 3, 6.1, {0.181, 0.262, 0.400}, 0.060, 0.050, 0},
+                                 {64, 128, 512, 2, 2.8, {0.250, 0.432, 0}, 0.101, 0.026, 3.4},
+                                 {128, 128, 512, 2, 3.2, {0.288, 0.557, 0}, 0.216, 0.001, 5.0},
+                                 {192, 128, 512, 2, 3.0, {0.429, 0.761, 0}, 0.322, 0, 6.5},
+                                 {32, 64, 128, 3, 5.5, {0.177, 0.262, 0.282}, 0.022, 0.052, 0}};
 // One 16-bit matrix (linear16.hip): 64 x 64, 128 x 64, 64 x 128, 128 x 128 (one
 // and two per CU), 256 x 128 and 256 x 256.
-constexpr ShapeCost kL16Cost[] = {{64, 64, 2, 2.0, {0.213, 0.368, 0}, 0, 0.138, 0.8},
-                                  {128, 64, 2, 3.2, {0.259, 0.533, 0}, 0.017, 0.126, 1.8},
-                                  {64, 128, 1, 1.2, {0.235, 0, 0}, 0.048, 0.164, 2.2},
-                                  {128, 128, 1, 1.5, {0.298, 0, 0}, 0.170, 0.126, 3.0},
-                                  {128, 128, 2, 2.4, {0.363, 0.433, 0}, 0.263, 0.085, 2.7},
-                                  {256, 128, 1, 0, {0.523, 0, 0}, 0.277, 0.011, 9.6},
-                                  {256, 256, 1, 0, {0.397, 0, 0}, 1.198, 0, 20.9}};
+constexpr ShapeCost kL16Cost[] = {{64, 64, 256, 2, 2.0, {0.213, 0.368, 0}, 0, 0.138, 0.8},
+                                  {128, 64, 256, 2, 3.2, {0.259, 0.533, 0}, 0.017, 0.126, 1.8},
+                                  {64, 128, 512, 1, 1.2, {0.235, 0, 0}, 0.048, 0.164, 2.2},
+                                  {128, 128, 512, 1, 1.5, {0.298, 0, 0}, 0.170, 0.126, 3.0},
+                                  {128, 128, 512, 2, 2.4, {0.363, 0.433, 0}, 0.263, 0.085, 2.7},
+                                  {256, 128, 512, 1, 0, {0.523, 0, 0}, 0.277, 0.011, 9.6},
+                                  {256, 256, 512, 1, 0, {0.397, 0, 0}, 1.198, 0, 20.9}};
+// 16-bit gate/up + SiLU-and-mul (gate_up_silu.hip): 64 x 64, 128 x 64, 128 x
+// 128, 192 x 128, 256 x 128 and 256 x 64.
+constexpr ShapeCost kGateUpCost[] = {{64, 64, 256, 2, 1.7, {0.328, 0.551, 0}, 0.055, 0.101, 0},
+                                     {128, 64, 256, 2, 3.6, {0.347, 0.715, 0}, 0.130, 0.038, 1.5},
+                                     {128, 128, 512, 1, 1.6, {0.655, 0, 0}, 0.277, 0.035, 2.7},
+                                     {192, 128, 512, 1, 1.3, {0.772, 0, 0}, 0.405, 0.007, 6.6},
+                                     {256, 128, 512, 1, 1.4, {0.889, 0, 0}, 0.650, 0, 8.6},
+                                     {256, 64, 512, 1, 0.1, {0.516, 0, 0}, 0.261, 0.068, 5.2}};
+// Int8 gate/up + SiLU-and-mul (w8a16.hip): 96 x 128, 64 x 64, 128 x 64 (three
+// and two per CU), 192 x 128, 256 x 128 and 128 x 64 in the step pipeline.
+constexpr ShapeCost kGateUp8Cost[] = {{96, 128, 256, 1, 2.8, {0.639, 0, 0}, 0.113, 0, 6.5},
+                                      {64, 64, 256, 3, 5.6, {0.250, 0.446, 0.644}, 0.092, 0.034, 2.7},
+                                      {128, 64, 256, 3, 4.4, {0.405, 0.570, 0.917}, 0.167, 0.025, 4.3},
+                                      {128, 64, 256, 2, 4.6, {0.382, 0.616, 0}, 0.179, 0.011, 5.4},
+                                      {192, 128, 512, 2, 0, {0.914, 2.080, 0}, 0.317, 0, 9.8},
+                                      {256, 128, 512, 1, 0, {0.888, 0, 0}, 0.747, 0, 10.5},
+                                      {128, 64, 256, 1, 0, {0.620, 0, 0}, 0.030, 0, 5.0}};
 
 }  // namespace tiled
 }  // namespace mi355

@@ -387,14 +387,6 @@ int w8_tiled(const W8Params& p, int shape, hipStream_t s) {
 // 128 x 64 (4 waves, 4 stages, one per CU).  Against the rounds rule before:
 // 1.5B 160 rows 39.1 -> 22.6 us, 256 rows 40.0 -> 28.2; 14B 100 rows 79.9 ->
 // 57.3; 7B 160 rows 104.5 -> 76.2.
-constexpr tiled::ShapeCost kGateUp8Cost[] = {{96, 128, 1, 2.8, {0.639, 0, 0}, 0.113, 0, 6.5},
-                                             {64, 64, 3, 5.6, {0.250, 0.446, 0.644}, 0.092, 0.034, 2.7},
-                                             {128, 64, 3, 4.4, {0.405, 0.570, 0.917}, 0.167, 0.025, 4.3},
-                                             {128, 64, 2, 4.6, {0.382, 0.616, 0}, 0.179, 0.011, 5.4},
-                                             {192, 128, 2, 0, {0.914, 2.080, 0}, 0.317, 0, 9.8},
-                                             {256, 128, 1, 0, {0.888, 0, 0}, 0.747, 0, 10.5},
-                                             {128, 64, 1, 0, {0.620, 0, 0}, 0.030, 0, 5.0}};
-
 template <typename T, typename TO>
 int w8_dual_shape(const W8Params& p, int shape, hipStream_t s) {
   constexpr int E = tiled::EPI_SILU_W8;
@@ -412,7 +404,7 @@ int w8_dual_shape(const W8Params& p, int shape, hipStream_t s) {
 template <typename T, typename TO>
 int w8_tiled_dual(const W8Params& p, hipStream_t s, int cus) {
   const double wmb = 2e-6 * static_cast<double>(p.n) * p.k;
-  return w8_dual_shape<T, TO>(p, tiled::plan_tiles(kGateUp8Cost, p.rows, p.n, p.k, wmb, cus, false).shape, s);
+  return w8_dual_shape<T, TO>(p, tiled::plan_tiles(tiled::kGateUp8Cost, p.rows, p.n, p.k, wmb, cus, false).shape, s);
 }
 
 // Small tiled shapes for 17 - 64 rows: 32 x 64 (2 waves) or, for n > 10000,
