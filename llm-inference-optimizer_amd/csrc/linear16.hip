@@ -155,15 +155,13 @@ int l16_tiled(const L16Params& p, int shape, hipStream_t s) {
   }
 }
 
-// Small tiled shapes: 32 x 64 (2 waves) or, for n > 10000, 32 x 128 (4 waves)
-// up to 32 rows; 64 x 64 (4 waves) up to 64; 4 stages.  From a sweep over
-// the Qwen2.5-1.5B / 7B down and o projections at 16 - 64 rows: on narrow
-// outputs (fewer than 128 tile columns) they lose to split-K weight
-// streaming (1.5B down, 32 rows: 38.0 vs 22.3 us).
+// Small tiled shapes for 17 - 64 rows (small_tiles_pay): 32 x 64 (2 waves), 32
+// x 128 (4 waves) and 64 x 64 (4 waves); 4 stages.  On narrow outputs they
+// lose to weight streaming here too (1.5B down, 32 rows: 38.0 vs 22.3 us).
 template <typename T, typename TO>
 int l16_tiled_small(const L16Params& p, hipStream_t s) {
   if (p.rows <= 32) {
-    if (p.n > 10000) return l16_tiled_cfg<T, TO, 1, 4, 1, 1, 4>(p, s);
+    if (tiled::small_tile_columns(p.rows, p.n) == 128) return l16_tiled_cfg<T, TO, 1, 4, 1, 1, 4>(p, s);
     return l16_tiled_cfg<T, TO, 1, 2, 1, 1, 4>(p, s);
   }
   return l16_tiled_cfg<T, TO, 2, 2, 1, 1, 4>(p, s);
@@ -197,8 +195,7 @@ int l16_typed(const L16Params& p, void* work, int64_t work_bytes, hipStream_t s,
     return tiled::split_k_launch<T, tiled::B_16, TO, tiled::EPI_LINEAR>(l16_tiled_params(p), sp,
                                                                          static_cast<float*>(work), s);
   if (p.rows <= 64) {
-    const int bn = (p.rows <= 32 && p.n > 10000) ? 128 : 64;
-    if (p.rows <= 16 || (p.n + bn - 1) / bn < 128)
+    if (!tiled::small_tiles_pay(p.rows, p.n))
       return w8_stream_launch<T, TO, false, 2>(w, l16_stream_plan(p.rows, p.k, p.n, cus), s);
     return l16_tiled_small<T, TO>(p, s);
   }

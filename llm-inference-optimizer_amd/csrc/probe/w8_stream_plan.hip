@@ -307,3 +307,13 @@ extern "C" __attribute__((visibility("default"))) double mi355_probe_tile_plan(i
     default: return run(kGateUp8Cost, 2.0, false);
   }
 }
+
+// Predicted us of the split plan (of no consequence where it does not split)
+// and, at 17 - 64 rows of wide outputs, of the unsplit kernel there (else 0).
+extern "C" __attribute__((visibility("default"))) void mi355_probe_split_cost(long long rows, long long k, long long n,
+                                                                               int wb, int cus, double* out2) {
+  using namespace mi355::tiled;
+  const uint32_t r = static_cast<uint32_t>(rows), kk = static_cast<uint32_t>(k), nn = static_cast<uint32_t>(n);
+  out2[0] = split_plan(r, kk, nn, wb, static_cast<uint32_t>(cus)).cost;
+  out2[1] = r > 16 && r <= 64 && nn > kWide ? wide_time(r, kk, nn, wb, static_cast<uint32_t>(cus)) : 0.0;
+}

@@ -107,6 +107,33 @@ constexpr TileCost kSplitCost8[SPLIT_TILES] = {
 // there): fixed us, us per MB of weights.
 constexpr double kStreamCost16[4][2] = {{3.1, 0.24}, {3.4, 0.29}, {4.1, 0.44}, {4.9, 0.52}};
 constexpr double kStreamCost8[4][2] = {{3.5, 0.36}, {4.1, 0.44}, {4.5, 0.69}, {4.9, 0.90}};
+// The kernels of 17 - 64 rows on outputs of more than kWide columns, which
+// those lines do not describe: the stream kernel at 17 - 24 and 25 - 32 rows,
+// then 32 x 64, 32 x 128 and 64 x 64 tiles (small_tiles_pay): fixed us, us per
+// K step of one and of more workgroups per CU, us per MB of weights and per MB
+// and row.  Fits of a sweep on MI355X over 36 outputs of 8192 - 32768 columns
+// (k 896 - 18944) at 17 - 64 rows, weights rotated through HBM: mean error 1 -
+// 6% per kernel.
+struct WideCost {
+  double c0, step1, step2, weight, row;
+};
+constexpr uint32_t kWide = 127 * 64;
+constexpr WideCost kWideCost16[5] = {{3.7, 0, 0, 0.152, 0.0025}, {4.8, 0, 0, 0.161, 0.0023},
+                                     {4.1, 0.246, 0.246, 0.016, 0.0006}, {0, 0.246, 0.246, 0.115, 0.0005},
+                                     {3.5, 0.217, 0.405, 0.051, 0.0007}};
+constexpr WideCost kWideCost8[5] = {{6.2, 0, 0, 0.171, 0.0043}, {7.9, 0, 0, 0.199, 0.0039},
+                                    {4.3, 0.236, 0.236, 0, 0.0001}, {2.0, 0.223, 0.223, 0.105, 0.0007},
+                                    {4.3, 0.222, 0.370, 0.023, 0.0010}};
+
+// Predicted us of the unsplit kernel of 17 - 64 rows of n > kWide columns.
+inline double wide_time(uint32_t rows, uint32_t k, uint32_t n, int wb, uint32_t cus) {
+  const uint32_t bn = small_tile_columns(rows, n);
+  int kind = rows <= 24 ? 0 : 1;
+  if (small_tiles_pay(rows, n)) kind = rows > 32 ? 4 : (bn == 64 ? 2 : 3);
+  const WideCost& c = wb == 1 ? kWideCost8[kind] : kWideCost16[kind];
+  const double wmb = static_cast<double>(n) * k * wb * 1e-6;
+  return c.c0 + (plan_cdiv(n, bn) <= cus ? c.step1 : c.step2) * plan_cdiv(k, 64u) + (c.weight + c.row * rows) * wmb;
+}
 
 // Whether 65 - 256 rows of an int8 product leave 32-row skinny tiles with split
 // K (w8a16.hip), which re-read the int8 weights per tile mostly from L2,
@@ -129,17 +156,26 @@ struct SplitPlan {
 // weight), against the fastest unsplit kernel at that size.  One workgroup
 // per CU: S = CUs / tiles, no more than 32, at least 4 K steps each, every
 // range with work.  Splitting has to win 3% and 1.5 us in the prediction (an
-// eager call also pays the second launch and the workspace on the host).
+// eager call also pays the second launch and the workspace on the host); on
+// wide outputs at 17 - 64 rows also 1% against the kernels that run there.
+// (The stream kernel's line alone split 86 int8 gate/up shapes that small
+// tiles run faster: 3584 -> 18944, 64 rows 30.8 us unsplit, 39.3 split; 1536
+// -> 8960, 64 rows 10.9 and 12.1.  What still splits: 5120 -> 13824 int8, 24
+// rows 28.0 -> 22.1, 64 rows 28.7 -> 26.0; 18944 -> 9000, 64 rows int8 83.8
+// -> 48.4, 16-bit 98.2 -> 67.4.  Over the sweep of 465 sizes the old line
+// split, two of the slower ones still do (0.8% and 1.4%; they were slower by up
+// to 2.0x), and 31 of the faster ones no longer do, by up to 13%.)
 inline SplitPlan split_plan(uint32_t rows, uint32_t k, uint32_t n, int wb, uint32_t cus) {
   const TileCost* sc = wb == 1 ? kSplitCost8 : kSplitCost16;
   const double wmb = static_cast<double>(n) * k * wb * 1e-6;
   SplitPlan best{-1, 1, 1e30, 0};
   if (rows <= 16) return best;
-  double direct;
+  double direct, wide = kNoLaunch;
   if (rows <= 64) {
     const int cls = rows <= 24 ? 0 : (rows <= 32 ? 1 : (rows <= 48 ? 2 : 3));
     const double* st = wb == 1 ? kStreamCost8[cls] : kStreamCost16[cls];
     direct = st[0] + st[1] * wmb;
+    if (n > kWide) wide = 0.99 * wide_time(rows, k, n, wb, cus);
   } else {
     const TilePlan unsplit = wb == 1 ? plan_tiles(kW8Cost, rows, n, k, wmb, cus, false)
                                      : plan_tiles(kL16Cost, rows, n, k, wmb, cus, false);
@@ -149,7 +185,12 @@ inline SplitPlan split_plan(uint32_t rows, uint32_t k, uint32_t n, int wb, uint3
     // 6.3, 3584 k 10.7, 4864 k 15.5)
     if (wb == 1 && w8_skinny_pays(rows, n) && 3.0 + 0.0023 * k < direct) direct = 3.0 + 0.0023 * k;
   }
-  const double limit = 0.97 * direct < direct - 1.5 ? 0.97 * direct : direct - 1.5;
+  const double margin = 0.97 * direct < direct - 1.5 ? 0.97 * direct : direct - 1.5;
+  const double limit = margin < wide ? margin : wide;
+  // 16-bit weight rows a multiple of 8 KiB apart, read by several ranges at
+  // once: 1.05 - 1.3x the prediction at 4096, 8192 and 12288 columns on wide
+  // outputs (4096 -> 16384, 17 rows: 28.3 predicted, 35.7 us measured)
+  const double strided = wide < kNoLaunch && wb == 2 && k % 4096 == 0 ? 1.15 : 1.0;
   const uint32_t steps = plan_cdiv(k, 64u);
   for (int t = 0; t < SPLIT_TILES; ++t) {
     const double fixed = sc[t].c0 + sc[t].weight * wmb;
@@ -166,7 +207,7 @@ inline SplitPlan split_plan(uint32_t rows, uint32_t k, uint32_t n, int wb, uint3
     const uint32_t per = plan_cdiv(steps, s);
     s = plan_cdiv(steps, per);
     if (s < 2) continue;
-    const double c = fixed + sc[t].step * per + sc[t].part * 8e-6 * s * rows * n;
+    const double c = strided * (fixed + sc[t].step * per + sc[t].part * 8e-6 * s * rows * n);
     if (c < best.cost && c < limit) best = SplitPlan{t, static_cast<int>(s), c, best.direct};
   }
   return best;

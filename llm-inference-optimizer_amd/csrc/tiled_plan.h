@@ -93,6 +93,18 @@ __attribute__((always_inline)) inline TilePlan plan_tiles(const ShapeCost (&tabl
   return best;
 }
 
+// Small tiles for 17 - 64 rows of the two linears: 32 x 64 or, for n > 10000,
+// 32 x 128 up to 32 rows, 64 x 64 above.  They read each weight byte once and x
+// once per workgroup, where skinny tiles re-load x for every weight piece or
+// the weights per 32-row tile, but only win with >= 128 tile columns to spread
+// over the CUs (a sweep over the Qwen2.5-1.5B / 7B projections at 16 - 64 rows:
+// int8 gate/up 7B, 32 rows 85.1 -> 40.7 us, 1.5B 21.3 -> 14.8 us; the 1536-wide
+// down and q/o projections 1.8x slower, so they keep weight streaming).
+inline uint32_t small_tile_columns(uint32_t rows, uint32_t n) { return rows <= 32 && n > 10000 ? 128u : 64u; }
+inline bool small_tiles_pay(uint32_t rows, uint32_t n) {
+  return rows > 16 && rows <= 64 && plan_cdiv(n, small_tile_columns(rows, n)) >= 128;
+}
+
 // One int8 matrix (w8a16.hip): 64 x 64, 64 x 128, 128 x 128, 192 x 128 (capped
 // at 128 registers, two per CU) and 32 x 64.
 constexpr ShapeCost kW8Cost[] = {{64, 64, 256, 3, 6.1, {0.181, 0.262, 0.400}, 0.060, 0.050, 0},

@@ -407,25 +407,13 @@ int w8_tiled_dual(const W8Params& p, hipStream_t s, int cus) {
   return w8_dual_shape<T, TO>(p, tiled::plan_tiles(tiled::kGateUp8Cost, p.rows, p.n, p.k, wmb, cus, false).shape, s);
 }
 
-// Small tiled shapes for 17 - 64 rows: 32 x 64 (2 waves) or, for n > 10000,
-// 32 x 128 (4 waves) up to 32 rows; 64 x 64 (4 waves) up to 64; 4 stages.
-// They read each weight byte once and x once per workgroup, where 24- or
-// 32-row skinny tiles re-load x for every weight piece and more rows re-read
-// the weights per 32-row tile -- but only win with >= 128 tile columns to
-// spread over the CUs (a sweep over the Qwen2.5-1.5B / 7B projections at 16 -
-// 64 rows: int8 gate/up 7B, 32 rows 85.1 -> 40.7 us, 1.5B 21.3 -> 14.8 us;
-// the 1536-wide down and q/o projections 1.8x slower, so they keep split-K
-// weight streaming).
-bool small_tiles_pay(int rows, int n) {
-  const int bn = (rows <= 32 && n > 10000) ? 128 : 64;
-  return rows > 16 && rows <= 64 && (n + bn - 1) / bn >= 128;
-}
-
+// Small tiled shapes for 17 - 64 rows (small_tiles_pay): 32 x 64 (2 waves), 32
+// x 128 (4 waves) and 64 x 64 (4 waves); 4 stages.
 template <typename T, typename TO, bool DUAL>
 int w8_tiled_small(const W8Params& p, hipStream_t s) {
   constexpr int EPI = DUAL ? tiled::EPI_SILU_W8 : tiled::EPI_W8;
   if (p.rows <= 32) {
-    if (p.n > 10000) return w8_tiled_cfg<T, TO, 1, 4, 1, 1, 4, EPI>(p, s);
+    if (tiled::small_tile_columns(p.rows, p.n) == 128) return w8_tiled_cfg<T, TO, 1, 4, 1, 1, 4, EPI>(p, s);
     return w8_tiled_cfg<T, TO, 1, 2, 1, 1, 4, EPI>(p, s);
   }
   return w8_tiled_cfg<T, TO, 2, 2, 1, 1, 4, EPI>(p, s);
@@ -464,7 +452,7 @@ int w8_typed(const W8Params& p, hipStream_t s, int cus, void* work = nullptr, in
   // (1.5B, 18 / 24 rows 15.46 / 15.50 -> 13.40 / 13.77 us; from 28 rows the
   // tiles lead, 15.53 vs 15.85, and at the 7B MLP, 20 rows 40.7 vs 45.8).
   const bool dual_stream = DUAL && p.rows <= 24 && p.k <= 2048;
-  if (small_tiles_pay(p.rows, p.n) && tiled_fits(p, DUAL) && !dual_stream) return w8_tiled_small<T, TO, DUAL>(p, s);
+  if (tiled::small_tiles_pay(p.rows, p.n) && tiled_fits(p, DUAL) && !dual_stream) return w8_tiled_small<T, TO, DUAL>(p, s);
   // 17 - 32 rows where the small tiles do not pay: the stream kernel with 6
   // or 8 x sets (1.5B down, 32 rows 20.6 -> 13.0 us; 7B down 44.4 -> 30.1;
   // 0.5B down 12.6 -> 7.3; the int8 gate/up + SiLU-and-mul, 0.5B 9.7 -> 8.9),

@@ -3,7 +3,8 @@ the probe library; no GPU call): over row counts, widths and depths of any
 alignment, a plan that splits gives every K range work, starts no more
 workgroups than the CUs, and wants a workspace of exactly its fp32 sums,
 bounded by one largest tile per CU; decode rows and wide outputs never split;
-sizes beyond any launch are answered, not divided by."""
+sizes beyond any launch are answered, not divided by; and wide outputs at 17 -
+64 rows split only where that is faster than the kernels that run there."""
 import ctypes
 import subprocess
 import sys
@@ -73,3 +74,37 @@ for rows in near:
 """
     res = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True)
     assert res.returncode == 0, (res.returncode, res.stderr)
+
+
+# (bytes per weight, rows, k, n) of wide outputs, us unsplit and split, measured on MI355X with weights from HBM
+WIDE_MEASURED = [
+    (1, 64, 1536, 8960, 10.8, 13.6), (1, 33, 1536, 8960, 10.4, 12.1), (1, 48, 2048, 11008, 12.7, 14.6),
+    (1, 64, 3584, 18944, 30.7, 39.6), (1, 33, 3584, 18944, 27.4, 35.5), (1, 40, 896, 32768, 11.7, 23.2),
+    (2, 64, 1536, 8960, 12.0, 13.9), (2, 40, 2048, 11008, 13.8, 14.8), (2, 32, 3584, 18944, 30.2, 38.5),
+    (2, 48, 3584, 18944, 37.6, 39.9), (2, 33, 5120, 13824, 29.3, 31.4), (2, 17, 4096, 12288, 23.9, 28.1),
+    (2, 33, 4096, 16384, 30.8, 36.3), (2, 17, 4096, 16384, 34.1, 35.8), (2, 33, 12288, 12288, 70.2, 74.9),
+    (1, 17, 5120, 13824, 25.4, 21.7), (1, 28, 5120, 13824, 31.5, 22.0), (1, 64, 5120, 13824, 28.7, 26.0),
+    (1, 17, 8192, 8192, 34.4, 18.5), (1, 64, 8192, 8192, 38.0, 22.5), (1, 17, 4096, 16384, 24.5, 18.8),
+    (2, 28, 5120, 13824, 39.2, 31.7), (2, 64, 8192, 8192, 43.5, 38.5), (2, 17, 18944, 9000, 84.5, 62.0),
+    (1, 64, 18944, 9000, 83.8, 48.4), (2, 64, 18944, 9000, 98.2, 67.4),
+]
+
+
+@pytest.mark.parametrize("wb,rows,k,n,unsplit,split", WIDE_MEASURED)
+def test_wide_outputs_split_where_it_measured_faster(plan, wb, rows, k, n, unsplit, split):
+    assert (plan(rows, k, n, wb, 256)[1] >= 0) == (split < unsplit)
+
+
+@pytest.mark.parametrize("wb", [1, 2])
+def test_wide_splits_beat_the_kernel_they_replace(plan, wb):
+    f = ctypes.CDLL(str(PROBE)).mi355_probe_split_cost
+    f.argtypes, f.restype = [ctypes.c_longlong] * 3 + [ctypes.c_int] * 2 + [ctypes.POINTER(ctypes.c_double)], None
+    out, splits = (ctypes.c_double * 2)(), 0
+    for k, n in [(896, 4864), (1536, 8960), (2048, 11008), (3584, 18944), (5120, 13824), (8192, 8192), (18944, 8200)]:
+        for rows in range(17, 65):
+            f(rows, k, n, wb, 256, out)
+            assert (out[1] > 0) == (n > 8128)
+            if plan(rows, k, n, wb, 256)[1] >= 0 and out[1] > 0:
+                splits += 1
+                assert out[0] <= 0.99 * out[1], (rows, k, n, *out)
+    assert splits > 0
