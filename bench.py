@@ -110,6 +110,7 @@ class Ctx:
         self.dev = torch.device("cuda:0")
         torch.cuda.set_device(self.dev)
         self.stream = torch.cuda.current_stream(self.dev).cuda_stream
+        self._scratch = None
         probe_path = ROOT / PKG / "libmi355_probe.so"
         self.probe = ctypes.CDLL(str(probe_path)) if probe_path.exists() else None
         if self.probe is not None:
@@ -213,30 +214,46 @@ class Ctx:
                 self.check("mi355_gate_up_silu_w8a16_fwd", st)
         return call
 
-    def w8a16_call(self, x, q, scale, out, bias=None):
+    def scratch(self, nbytes):
+        """`nbytes` of device scratch for the linears' split K, shared by every
+        call on the stream (their kernels run in order): (tensor, address)."""
+        if nbytes <= 0:
+            return None, None
+        if self._scratch is None or self._scratch.numel() < nbytes:
+            self._scratch = self.torch.empty(nbytes, dtype=self.torch.uint8, device=self.dev)
+        return self._scratch, self._scratch.data_ptr()
+
+    def w8a16_call(self, x, q, scale, out, bias=None, split=True):
+        """The int8 linear as the package calls it, with the workspace its
+        split-K kernels ask for; split=False: its unsplit kernels."""
         M, K = x.shape
         N = q.shape[0]
         code = self.L.DTYPE_CODE[x.dtype]
-        f = self.lib.mi355_w8a16_linear_fwd
+        f = self.lib.mi355_w8a16_linear_ws_fwd
+        nbytes = self.lib.mi355_w8a16_linear_workspace(M, K, N) if split else 0
+        work, wp = self.scratch(nbytes)
         args = (x.data_ptr(), q.data_ptr(), scale.data_ptr(), bias.data_ptr() if bias is not None else None,
                 out.data_ptr(), M, K, N, K, K, N, code, self.L.DTYPE_CODE[scale.dtype],
-                self.L.DTYPE_CODE[bias.dtype] if bias is not None else 0, code)
+                self.L.DTYPE_CODE[bias.dtype] if bias is not None else 0, code, wp, nbytes)
 
-        def call():
+        def call(keep=work):
             st = f(*args, self.stream)
             if st:
                 self.check("mi355_w8a16_linear_fwd", st)
         return call
 
-    def linear16_call(self, x, w, out, bias=None):
+    def linear16_call(self, x, w, out, bias=None, split=True):
+        """The 16-bit linear, with the workspace rule of w8a16_call."""
         M, K = x.shape
         N = w.shape[0]
         code = self.L.DTYPE_CODE[x.dtype]
-        f = self.lib.mi355_linear16_fwd
+        f = self.lib.mi355_linear16_ws_fwd
+        nbytes = self.lib.mi355_linear16_workspace(M, K, N) if split else 0
+        work, wp = self.scratch(nbytes)
         args = (x.data_ptr(), w.data_ptr(), bias.data_ptr() if bias is not None else None, out.data_ptr(),
-                M, K, N, K, K, N, code, self.L.DTYPE_CODE[bias.dtype] if bias is not None else 0, code)
+                M, K, N, K, K, N, code, self.L.DTYPE_CODE[bias.dtype] if bias is not None else 0, code, wp, nbytes)
 
-        def call():
+        def call(keep=work):
             st = f(*args, self.stream)
             if st:
                 self.check("mi355_linear16_fwd", st)
@@ -545,55 +562,50 @@ KNOWN_LAUNCHES = {
     ("w8a16_stream<mi355::BF16, mi355::BF16, 4, 2, 1, true, 1>", 1184 * 64 * 1): (
         "int8 gate/up + SiLU-and-mul 7B, 8 rows, 2 x [18944,3584] int8, bf16",
         2 * 18944 * 3584 + 8 * 18944 + 8 * 3584 * 2 + 8 * 18944 * 2),
-    # the stream kernel at 32 - 64 rows (bench.py --only decode-wide-rows), at their launch plans
+    # 32 - 64 rows (bench.py --only decode-wide-rows): the stream kernel at 32 rows of the 1.5B
+    # down projection, split K (first pass; then split_k_reduce) for the 7B one
     ("w8a16_stream<mi355::F16, mi355::F16, 2, 8, 1, false, 1>", 256 * 64 * 8): (
         "W8A16 1.5B down, 32 rows, [1536,8960] int8, fp16", 1536 * 8960 + 4 * 1536 + 32 * 8960 * 2 + 32 * 1536 * 2),
-    ("w8a16_stream<mi355::BF16, mi355::BF16, 2, 12, 1, false, 1>", 448 * 64 * 4): (
-        "W8A16 7B down, 48 rows, [3584,18944] int8, bf16",
-        3584 * 18944 + 4 * 3584 + 48 * 18944 * 2 + 48 * 3584 * 2),
     ("w8a16_stream<mi355::F16, mi355::F16, 2, 8, 1, false, 2>", 256 * 64 * 8): (
         "16-bit linear, 32 rows, [1536,8960] weights, fp16 (1.5B down)",
         1536 * 8960 * 2 + 32 * 8960 * 2 + 32 * 1536 * 2),
-    ("w8a16_stream<mi355::BF16, mi355::BF16, 2, 16, 1, false, 2>", 448 * 64 * 4): (
-        "16-bit linear, 64 rows, [3584,18944] weights, bf16 (7B down)",
-        3584 * 18944 * 2 + 64 * 18944 * 2 + 64 * 3584 * 2),
     ("w8a16_stream<mi355::F16, mi355::F16, 2, 2, 2, false, 2>", 256 * 64 * 8): (
         "16-bit linear, 8 rows, [1536,8960] weights, fp16 (1.5B down)", 1536 * 8960 * 2 + 8 * 8960 * 2 + 8 * 1536 * 2),
     ("w8a16_stream<mi355::BF16, mi355::BF16, 4, 2, 1, false, 2>", 224 * 64 * 8): (
         "16-bit linear, 8 rows, [3584,18944] weights, bf16 (7B down)", 3584 * 18944 * 2 + 8 * 18944 * 2 + 8 * 3584 * 2),
-    # MFMA-bound prefill GEMMs: (label, algorithmic bytes, flops)
-    # (the 1.5B gate/up at 1024 and 4096 rows runs as a column split: whole
-    # rounds of 256 x 128 tiles over the first 8192 columns, then 768 columns)
-    ("tiled_gemm<mi355::F16, 0, mi355::F16, 2, 4, 4, 1, 1, 2, 1, 0, 0>", 256 * 512): (
+    # tiled GEMMs: (label, algorithmic bytes, flops).  The first passes of split K write fp32
+    # sums of 9 K ranges (64 x 128 tiles) or 2 (128 x 128 tiles)
+    ("tiled_gemm<mi355::BF16, 1, mi355::F32, 1, 4, 2, 1, 4, 4, 1, 0, 4>", 28 * 9 * 256): (
+        "W8A16 7B down, 48 rows, [3584,18944] int8, bf16 (split K, first pass)",
+        3584 * 18944 + 48 * 18944 * 2 + 9 * 48 * 3584 * 4, 2 * 48 * 18944 * 3584),
+    ("tiled_gemm<mi355::BF16, 0, mi355::F32, 1, 4, 2, 1, 4, 4, 1, 0, 4>", 28 * 9 * 256): (
+        "16-bit linear, 64 rows, [3584,18944] weights, bf16 (7B down; split K, first pass)",
+        3584 * 18944 * 2 + 64 * 18944 * 2 + 9 * 64 * 3584 * 4, 2 * 64 * 18944 * 3584),
+    ("tiled_gemm<mi355::F16, 1, mi355::F32, 2, 4, 2, 1, 4, 3, 1, 0, 3>", 96 * 2 * 512): (
+        "W8A16 prefill down, 1024 rows, [1536,8960] int8, fp16 (split K, first pass)",
+        1536 * 8960 + 1024 * 8960 * 2 + 2 * 1024 * 1536 * 4, 2 * 1024 * 8960 * 1536),
+    # the 1.5B gate/up at 1024 and 4096 rows runs as a column split: whole rounds of 256 x 128
+    # tiles over the first 8192 columns, then 768 columns in 64 x 64 or 256 x 64 tiles
+    ("tiled_gemm<mi355::F16, 0, mi355::F16, 2, 4, 4, 1, 1, 2, 1, 0, 3>", 256 * 512): (
         "gate/up + SiLU-and-mul prefill, 1024 rows, first 8192 of 8960 columns, fp16",
         2 * 8192 * 1536 * 2 + 1024 * 1536 * 2 + 1024 * 8192 * 2, 4 * 1024 * 1536 * 8192),
-    ("tiled_gemm<mi355::F16, 0, mi355::F16, 2, 2, 1, 1, 1, 4, 0, 0, 0>", 192 * 256): (
+    ("tiled_gemm<mi355::F16, 0, mi355::F16, 2, 2, 1, 1, 1, 3, 1, 0, 3>", 192 * 256): (
         "gate/up + SiLU-and-mul prefill, 1024 rows, last 768 of 8960 columns, fp16",
         2 * 768 * 1536 * 2 + 1024 * 1536 * 2 + 1024 * 768 * 2, 4 * 1024 * 1536 * 768),
-    ("tiled_gemm<mi355::F16, 0, mi355::F16, 2, 4, 4, 1, 1, 2, 1, 0, 0>", 1024 * 512): (
+    ("tiled_gemm<mi355::F16, 0, mi355::F16, 2, 4, 4, 1, 1, 2, 1, 0, 3>", 1024 * 512): (
         "gate/up + SiLU-and-mul prefill, 4096 rows, first 8192 of 8960 columns, fp16",
         2 * 8192 * 1536 * 2 + 4096 * 1536 * 2 + 4096 * 8192 * 2, 4 * 4096 * 1536 * 8192),
-    ("tiled_gemm<mi355::F16, 0, mi355::F16, 2, 2, 2, 1, 1, 2, 1, 0, 0>", 384 * 256): (
+    ("tiled_gemm<mi355::F16, 0, mi355::F16, 4, 2, 2, 1, 1, 3, 0, 0, 3>", 192 * 512): (
         "gate/up + SiLU-and-mul prefill, 4096 rows, last 768 of 8960 columns, fp16",
         2 * 768 * 1536 * 2 + 4096 * 1536 * 2 + 4096 * 768 * 2, 4 * 4096 * 1536 * 768),
-    ("tiled_gemm<mi355::F16, 1, mi355::F16, 2, 2, 2, 1, 0, 2, 1, 0, 0>", 1120 * 256): (
-        "W8A16 prefill gate/up, 1024 rows, [8960,1536] int8, fp16",
-        8960 * 1536 + 4 * 8960 + 1024 * 1536 * 2 + 1024 * 8960 * 2, 2 * 1024 * 1536 * 8960),
-    ("tiled_gemm<mi355::F16, 1, mi355::F16, 2, 2, 1, 1, 0, 4, 0, 0, 0>", 384 * 256): (
-        "W8A16 prefill down, 1024 rows, [1536,8960] int8, fp16",
-        1536 * 8960 + 4 * 1536 + 1024 * 8960 * 2 + 1024 * 1536 * 2, 2 * 1024 * 8960 * 1536),
-    # narrow outputs filling half to all of the CUs: 64 x 128 tiles of 8 waves (the
-    # 1024-row q/o projection launches the same grid; its launches mix into this row)
-    ("tiled_gemm<mi355::F16, 1, mi355::F16, 2, 4, 1, 1, 0, 4, 1, 0, 0>", 192 * 512): (
-        "W8A16 prefill down, 1024 rows, [1536,8960] int8, fp16 (64x128 tiles)",
-        1536 * 8960 + 4 * 1536 + 1024 * 8960 * 2 + 1024 * 1536 * 2, 2 * 1024 * 8960 * 1536),
-    # the wide-output plan from 1024 rows: 128 x 128 tiles of 8 waves, 3-stage ring
-    # (at 1024 rows its 560 tiles would take two rounds of 512 slots: there the
-    # 192 x 128 tile of 8 waves, registers capped for two workgroups per CU)
-    ("tiled_gemm<mi355::F16, 1, mi355::F16, 2, 4, 3, 1, 0, 2, 1, 4, 1>", 420 * 512): (
+    # one int8 matrix, unsplit, by the tile plan
+    ("tiled_gemm<mi355::F16, 1, mi355::F16, 1, 2, 1, 1, 0, 4, 0, 0, 4>", 768 * 128): (
+        "W8A16 prefill q/o, 1024 rows, [1536,1536] int8, fp16 (32x64 tiles)",
+        1536 * 1536 + 4 * 1536 + 1024 * 1536 * 2 + 1024 * 1536 * 2, 2 * 1024 * 1536 * 1536),
+    ("tiled_gemm<mi355::F16, 1, mi355::F16, 2, 4, 3, 1, 0, 2, 1, 4, 2>", 420 * 512): (
         "W8A16 prefill gate/up, 1024 rows, [8960,1536] int8, fp16 (192x128 tiles)",
         8960 * 1536 + 4 * 8960 + 1024 * 1536 * 2 + 1024 * 8960 * 2, 2 * 1024 * 1536 * 8960),
-    ("tiled_gemm<mi355::F16, 1, mi355::F16, 2, 4, 2, 1, 0, 3, 1, 0, 0>", 2240 * 512): (
+    ("tiled_gemm<mi355::F16, 1, mi355::F16, 2, 4, 2, 1, 0, 3, 1, 0, 3>", 2240 * 512): (
         "W8A16 prefill gate/up, 4096 rows, [8960,1536] int8, fp16 (128x128 tiles)",
         8960 * 1536 + 4 * 8960 + 4096 * 1536 * 2 + 4096 * 8960 * 2, 2 * 4096 * 1536 * 8960),
 }
@@ -1036,7 +1048,7 @@ def run_only(ctx, args, sets):
             log(json.dumps(bench_w8a16(ctx, shapes=[s for s in W8A16_SHAPES if s[0] == 8 and s[4] in
                                                     ("gate/up proj", "down proj", "7b gate/up proj", "7b down proj")],
                                        iters=iters, baselines=False)))
-    elif args.only == "decode-wide-rows":  # kernel only: the stream kernel at 32 - 64 rows (for PMC runs)
+    elif args.only == "decode-wide-rows":  # kernels only: down projections at 32 - 64 rows (for PMC runs)
         del sets
         torch.cuda.empty_cache()
         log(json.dumps(bench_w8a16(ctx, shapes=[(32, 8960, 1536, "f16", "down proj"),
@@ -1663,7 +1675,7 @@ def _stream_sweep_shape(ctx, tag, label, M, nchunk, dual, wb, wide16, o, ref, li
             bad.append((rpw, r4, waves, u, err))
         spin_up(ctx, calls, ms=3.0)
         res[f"rpw{rpw}_w{waves}_u{u}"] = round(time_graph(ctx, calls, nodes, replays=5), 3)
-    # the library's own launch last, on a device already warm from the
+    # the library's own launch (unsplit, as the shapes) last, on a device already warm from the
     # shapes (timed first it read 3-10% high: clocks still ramping)
     spin_up(ctx, lib_calls, ms=5.0)
     res["library_us"] = round(time_graph(ctx, lib_calls, nodes, replays=5), 3)
@@ -1706,8 +1718,8 @@ def w8_stream_sweep(ctx, shapes=W8_STREAM_SWEEP_SHAPES, wide16=False, rpws=(4, 6
             lib_calls = [ctx.gate_up_w8_call(x, q[0], sc[0], q[1], sc[1], o) for q, sc in zip(qs, scs)]
             ctx.gate_up_w8_call(x, qs[0][0], scs[0][0], qs[0][1], scs[0][1], ref)()
         else:
-            lib_calls = [ctx.w8a16_call(x, q[0], sc[0], o) for q, sc in zip(qs, scs)]
-            ctx.w8a16_call(x, qs[0][0], scs[0][0], ref)()
+            lib_calls = [ctx.w8a16_call(x, q[0], sc[0], o, split=False) for q, sc in zip(qs, scs)]
+            ctx.w8a16_call(x, qs[0][0], scs[0][0], ref, split=False)()
         torch.cuda.synchronize()
 
         def make_calls(rpw, r4, waves, u, x=x, qs=qs, scs=scs, o=o, dual=dual):
@@ -1755,8 +1767,8 @@ def l16_stream_sweep(ctx, shapes=L16_SWEEP_SHAPES, rpws=(4, 6, 8, 12, 16)):
         x = rand(ctx, (M, K), 3200 + M, F16)
         o = torch.empty((M, N), dtype=F16, device=ctx.dev)
         ref = torch.empty_like(o)
-        lib_calls = [ctx.linear16_call(x, w, o) for w in ws]
-        ctx.linear16_call(x, ws[0], ref)()
+        lib_calls = [ctx.linear16_call(x, w, o, split=False) for w in ws]
+        ctx.linear16_call(x, ws[0], ref, split=False)()
         torch.cuda.synchronize()
         out[label] = _stream_sweep_shape(
             ctx, "l16", label, M, -(-K // 128), False, 2, True, o, ref, lib_calls,
@@ -2151,7 +2163,8 @@ LINEAR16_SHAPES = [(1, 8960, 1536, "f16", "qwen2.5-1.5b down"), (8, 8960, 1536, 
 
 def bench_linear16(ctx, shapes=LINEAR16_SHAPES, iters=300, baselines=True):
     """The MLP's down projection at decode rows on the HIP 16-bit linear
-    (mi355_linear16_fwd, weight streaming on MFMA) against torch's linear
+    (mi355_linear16_ws_fwd: weight streaming on MFMA, from 17 rows split K)
+    against torch's linear
     (hipBLASLt), the call FusedMLP makes otherwise, on per-layer weight sets
     whose footprint exceeds 1 GiB (cold HBM, as a decode step walking the
     layers).  Algorithmic bytes: weights + x + out.  Timed over back-to-back
@@ -2174,8 +2187,10 @@ def bench_linear16(ctx, shapes=LINEAR16_SHAPES, iters=300, baselines=True):
         best = min(us, us_graph)
         key = f"{label}_M{M}_{dname}"
         small_tiles = 16 < M <= 64 and -(-N // (128 if (M <= 32 and N > 10000) else 64)) >= 128
-        entry = kernel_entry("w8a16_stream (16-bit weights)" if M <= 64 and not small_tiles else "linear16 tiled",
-                             nbytes, best,
+        kname = "w8a16_stream (16-bit weights)" if M <= 64 and not small_tiles else "linear16 tiled"
+        if ctx.lib.mi355_linear16_workspace(M, K, N) > 0:
+            kname = "linear16 tiled (split K) + split_k_reduce"
+        entry = kernel_entry(kname, nbytes, best,
                              {"rows": M, "k": K, "n": N, "weight_sets": layers, "eager_us": round(us, 3),
                               "graph_us": round(us_graph, 3)})
         if (M, K, N, dname) == (8, 8960, 1536, "f16"):
@@ -2194,23 +2209,28 @@ def bench_linear16(ctx, shapes=LINEAR16_SHAPES, iters=300, baselines=True):
     return res
 
 
-def w8a16_kernel_name(M, N, K=0):
-    """The kernel mi355_w8a16_linear_fwd runs for this shape (aligned inputs,
-    descriptors that fit): the weight-streaming kernel up to 48 rows, but
-    for wide outputs with 2048 < k < 3072 beyond 8 rows (the skinny split-K
-    kernel) and where the small tiled shapes pay (17 - 64 rows, >= 128 tile
-    columns); the skinny kernel for small grids, the tiled MFMA GEMM
-    otherwise."""
+def w8a16_kernel_name(M, N, K=0, workspace=0):
+    """The kernel mi355_w8a16_linear_ws_fwd runs for this shape (aligned
+    inputs, descriptors that fit), given the workspace bytes it asks for: split
+    K where it asks for any; the weight-streaming kernel up to 48 rows (64 for
+    at most 8 MB of weights), but for wide outputs with 2048 < k < 3072 beyond
+    8 rows (the skinny kernel) and where the small tiled shapes pay (17 - 64
+    rows, >= 128 tile columns); the skinny kernel for small grids, the tiled
+    MFMA GEMM otherwise."""
+    if workspace > 0:
+        return "tiled_gemm<int8 B> (split K) + split_k_reduce"
     bn = 128 if (M <= 32 and N > 10000) else 64
     if 16 < M <= 64 and -(-N // bn) >= 128:
         return "tiled_gemm<int8 B> (small tiles)"
-    if M <= 8 or (M <= 48 and not (N > 10000 and 2048 < K < 3072)):
+    if M <= 8 or ((M <= 48 or (M <= 64 and N * K <= 8 << 20)) and not (N > 10000 and 2048 < K < 3072)):
         return "w8a16_stream"
     if M <= 32:
         return "w8a16_skinny"
     tiles64 = ((N + 63) // 64) * ((M + 63) // 64)
     skinny = M <= 256 and (tiles64 < 32 or (M <= 128 and N < 2048))
     return "w8a16_skinny" if skinny else "tiled_gemm<int8 B>"
+
+
 MFMA_PEAK_TFLOPS = 2500.0  # MI355X dense fp16 / bf16
 
 
@@ -2238,7 +2258,7 @@ def bench_w8a16(ctx, shapes=W8A16_SHAPES, iters=300, baselines=True):
         spin_up(ctx, calls)
         us = time_loop(ctx, calls, iters)
         us_graph = time_graph(ctx, calls, max(2 * sets, 64) if sets <= 256 else sets)
-        kname = w8a16_kernel_name(M, N, K)
+        kname = w8a16_kernel_name(M, N, K, ctx.lib.mi355_w8a16_linear_workspace(M, K, N))
         entry = kernel_entry(kname, nbytes, min(us, us_graph),
                              {"layer": label, "M": M, "K": K, "N": N, "dtype": dname, "weight_sets": sets,
                               "eager_us": round(us, 3), "graph_us": round(us_graph, 3),
@@ -2273,7 +2293,7 @@ def bench_prefill_core(ctx, shapes=((1024, 1536, 8960), (1024, 8960, 1536), (409
                                       (4096, 8960, 1536)), iters=200):
     """The tiled GEMM core at prefill rows with each kind of B operand, next
     to hipBLASLt: the 1.5B gate/up and down projections (fp16 x) through
-    mi355_linear16_fwd (16-bit weights), mi355_w8a16_linear_fwd (int8 weights,
+    mi355_linear16_ws_fwd (16-bit weights), mi355_w8a16_linear_ws_fwd (int8 weights,
     widened after each LDS read) and torch.matmul on the 16-bit weights.  If
     widening the int8 weights were what held the W8A16 GEMM back, the 16-bit
     path of the same core would be the faster one.  Cold weights (rotating

@@ -5,11 +5,14 @@ import csv
 import importlib
 import importlib.util
 import re
+import shutil
 import subprocess
 import sys
 from pathlib import Path
 
 import pytest
+
+from test_tile_plan_cpu import GATE_UP16, PROBE, W8, split_plan, tile_plan
 
 ROOT = Path(__file__).resolve().parents[1]
 
@@ -65,6 +68,64 @@ def test_stream_kernel_fragments_name_every_template_argument(bench):
     assert frags
     for frag in frags:
         assert len(frag[len("w8a16_stream<"):-1].split(",")) == arity, frag
+
+
+@pytest.fixture(scope="module")
+def kernel_names():
+    """The demangled names of the kernels the library registers, as a trace lists them."""
+    lib = ROOT / "llm-inference-optimizer_amd" / "libmi355_fused.so"
+    if not lib.exists() or shutil.which("c++filt") is None:
+        pytest.skip("needs the built library and c++filt")
+    mangled = sorted(set(re.findall(rb"_ZN5mi355[0-9A-Za-z_]*(?:tiled_gemm|w8a16_stream|rmsnorm_|silu_mul_)[0-9A-Za-z_]*",
+                                    lib.read_bytes())))
+    out = subprocess.run(["c++filt"], input=b"\n".join(mangled), capture_output=True, check=True).stdout
+    return out.decode()
+
+
+def test_known_launches_name_kernels_of_the_library(bench, kernel_names):
+    """A fragment that matches no kernel leaves its row out of every summary."""
+    for frag, _ in bench.KNOWN_LAUNCHES:
+        if frag != "stream_copy":  # the probe library's
+            assert frag in kernel_names, frag
+
+
+def test_known_tiled_launches_are_those_the_plans_take(bench):
+    """The grid of each prefill label is that of the plan at its sizes (256 CUs)."""
+    if not PROBE.exists():
+        pytest.skip("probe library not built")
+
+    def wgs(rows, cols, shape):
+        return -(-rows // shape[0]) * -(-cols // shape[1]) * shape[2]
+
+    grids = {}
+    for rows in (1024, 4096):
+        _, _, lead, _, a, b = tile_plan(GATE_UP16, rows, 1536, 8960)
+        assert lead == 8192
+        grids[f"gate/up + SiLU-and-mul prefill, {rows} rows, first 8192"] = wgs(rows, lead, a)
+        grids[f"gate/up + SiLU-and-mul prefill, {rows} rows, last 768"] = wgs(rows, 8960 - lead, b)
+        assert split_plan(rows, 1536, 8960, 1)[0] < 0
+        grids[f"W8A16 prefill gate/up, {rows} rows"] = wgs(rows, 8960, tile_plan(W8, rows, 1536, 8960)[4])
+    assert split_plan(1024, 1536, 1536, 1)[0] < 0
+    grids["W8A16 prefill q/o, 1024 rows"] = wgs(1024, 1536, tile_plan(W8, 1024, 1536, 1536)[4])
+    for label, wb, threads, rows, k, n in (("W8A16 7B down, 48 rows", 1, 256, 48, 18944, 3584),
+                                           ("16-bit linear, 64 rows", 2, 256, 64, 18944, 3584),
+                                           ("W8A16 prefill down, 1024 rows", 1, 512, 1024, 8960, 1536)):
+        tile, splits, bm, bn = split_plan(rows, k, n, wb)
+        assert tile >= 0, label
+        grids[label] = wgs(rows, n, (bm, bn, threads)) * splits
+    known = {v[0]: grid for (frag, grid), v in bench.KNOWN_LAUNCHES.items() if frag.startswith("tiled_gemm<")}
+    assert len(known) == len(grids)
+    for label, grid in grids.items():
+        assert [g for name, g in known.items() if name.startswith(label)] == [grid], label
+
+
+def test_kernel_names_of_the_w8a16_table(bench):
+    """With a workspace the narrow deep products split; without one they do not."""
+    assert bench.w8a16_kernel_name(64, 3584, 18944, 1) == "tiled_gemm<int8 B> (split K) + split_k_reduce"
+    assert bench.w8a16_kernel_name(64, 1536, 1536) == "w8a16_stream"  # at most 8 MB
+    assert bench.w8a16_kernel_name(64, 1536, 8960) == "w8a16_skinny"
+    assert bench.w8a16_kernel_name(64, 8960, 1536) == "tiled_gemm<int8 B> (small tiles)"
+    assert bench.w8a16_kernel_name(1024, 8960, 1536) == "tiled_gemm<int8 B>"
 
 
 def _write(path, rows):

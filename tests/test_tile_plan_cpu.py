@@ -20,6 +20,16 @@ def tile_plan(table, rows, k, n, cus=256):
     return us, out[0], out[1], out[2], tuple(out[3:6]), tuple(out[6:9])
 
 
+def split_plan(rows, k, n, wb, cus=256):
+    """(tile (< 0: not split), K ranges, the tile's rows, its columns)"""
+    f = ctypes.CDLL(str(PROBE)).mi355_probe_split_plan
+    f.argtypes = [ctypes.c_longlong] * 3 + [ctypes.c_int] * 2 + [ctypes.POINTER(ctypes.c_int)]
+    f.restype = ctypes.c_longlong
+    out = (ctypes.c_int * 4)()
+    f(rows, k, n, wb, cus, out)
+    return tuple(out)
+
+
 def _threads(rows, cols, shape):
     bm, bn, threads = shape
     return -(-rows // bm) * -(-cols // bn) * threads
