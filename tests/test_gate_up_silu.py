@@ -81,11 +81,11 @@ def _check_vs_oracle(orc, got16, got32, x, wg, wu, dt):
     # 9 - 16 rows: 4-row workgroups where 8-row ones would number under 4 per
     # CU (ragged last workgroup), 16-row ones of about 5 waves per CU from k = 2048
     (10, 896, 4874, F16), (12, 2048, 11008, BF16),
-    # prefill rows: the tiled GEMM (each of its three launch shapes, k tails, ragged edges)
+    # prefill rows: the tiled GEMM (64 x 64 and, at 200 rows, 128 x 128 tiles; k tails, ragged edges)
     (64, 1536, 1000, F16), (200, 640, 10240, BF16), (300, 1552, 520, F16), (257, 96, 333, BF16),
     # 17 - 64 rows: the small tiled shapes (32 x 64, 32 x 128 for n_out > 10000, 64 x 64)
     (20, 256, 16400, BF16), (24, 1536, 8960, F16), (40, 256, 4000, F16), (63, 136, 72, BF16),
-    # > 128 rows, few tiles: 256 x 64 (main loop and k tail; tail only)
+    # > 128 rows, few tiles (main loop and k tail; tail only)
     (1100, 1000, 300, F16), (1030, 72, 130, BF16),
 ])
 def test_gate_up_silu_matches_oracle(pkg, orc, cuda, rows, k, n, dt):
@@ -132,7 +132,7 @@ def test_strided_views_and_3d_input_give_identical_bits(pkg, cuda):
     assert torch.equal(pkg.fused_gate_up_silu(x, wg, wu), want)   # run to run
 
 
-@pytest.mark.parametrize("rows,k,n", [(5, 256, 48), (1024, 64, 8960)])  # decode rows; a column split
+@pytest.mark.parametrize("rows,k,n", [(5, 256, 48), (1024, 64, 8960)])  # decode rows; 64 x 64 tiles
 def test_out_row_stride_through_abi(pkg, cuda, rows, k, n):
     """Writing into a row-strided output leaves the gaps untouched."""
     L = importlib.import_module("llm-inference-optimizer_amd._lib")
@@ -221,12 +221,9 @@ def test_large_shape_against_torch_fp64(pkg, cuda):
 
 @pytest.mark.parametrize("rows,k,n,dt", [
     (1024, 1536, 8960, F16), (2048, 3584, 4736, BF16),
-    # ragged rows, k and n on the sub-step ring: 128 x 64 tiles two per CU,
-    # then 256 x 128 tiles, then a column split (6528 columns in 256 x 128
-    # tiles, the last 72 in 64 x 64)
+    # (both column splits.)  Ragged rows, k and n on 64 x 64 tiles
     (300, 264, 8200, BF16), (520, 264, 8000, F16), (1030, 264, 6600, F16),
-    # whole rounds that end inside a 128-column block: 768 tiles of 256 x 128
-    # over 16384 columns (6 row blocks), then 2560 columns of 128 x 64 tiles
+    # 128 x 64 tiles, two per CU
     (1536, 264, 18944, BF16),
 ])
 def test_prefill_shapes_against_torch_fp64(pkg, cuda, rows, k, n, dt):
@@ -254,10 +251,10 @@ def test_prefill_shapes_against_torch_fp64(pkg, cuda, rows, k, n, dt):
 
 def test_tiled_launch_shapes_agree_bitwise(pkg, cuda):
     """Every tiled launch shape (33 .. 1536 rows of the 1.5B MLP: 64 x 64,
-    128 x 64 on 4 stages and on the sub-step ring, 256 x 64, 256 x 128 on the
-    ring, and the column splits at 1024 and 1025 rows) adds the k products in
-    the same order, so a prefix of the rows gives the same bits whichever
-    shape runs."""
+    128 x 64, 256 x 64, 128 x 128 and column splits of 192 x 128 and 256 x 128
+    tiles, at 1025 and 1536 rows with larger tiles behind them) adds the k
+    products in the same order, so a prefix of the rows gives the same bits
+    whichever shape runs."""
     torch.manual_seed(5)
     k, n = 1536, 8960
     x = torch.randn(1536, k, device=cuda).to(F16)

@@ -155,8 +155,8 @@ def test_graph_replays_match_eager(pkg, cuda, rows, k, n):
 
 @pytest.mark.parametrize("rows,k,n,dt", [
     (2048, 3584, 4736, BF16),   # 128 x 64 tiles on the sub-step ring
-    (1024, 1536, 18944, BF16),  # 256 x 128 tiles on the ring
-    (1030, 272, 18900, F16),    # 256 x 128, ragged rows and n, k tail
+    (1024, 1536, 18944, BF16),
+    (1030, 272, 18900, F16),    # ragged rows and n, k tail
 ])
 def test_prefill_shape_against_torch_fp64(pkg, cuda, rows, k, n, dt):
     x, qg, sg, qu, su = _inputs(rows, k, n, dt, 21, cuda, pkg)

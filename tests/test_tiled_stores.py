@@ -3,7 +3,9 @@ through LDS where the output's row stride and address allow 16-byte stores,
 8-byte stores or single elements otherwise, ragged last segments and rows in
 each.  The same call into outputs of those four kinds through the C ABI gives
 the same values (equal bits: one kernel, one summation order), and nothing
-outside the output's columns is written."""
+outside the output's columns is written.  The small sizes run 64 x 64 tiles
+(int8 also 32 x 64); TILE_CASES names a size for every other tile of the two
+linears (test_tile_plan_cpu.py checks that it takes it)."""
 import importlib
 
 import pytest
@@ -29,13 +31,29 @@ def _call(lib, int8, x, w, scale, bias, out, os, n):
                                   0 if bias is None else CODE[bias.dtype], CODE[out.dtype], stream)
 
 
+# (int8 weights, tile, rows, n, k)
+TILE_CASES = [(False, (128, 64), 67, 12099, 1872), (False, (64, 128), 66, 8237, 1872),
+              (False, (128, 128), 67, 16450, 1872), (False, (256, 128), 130, 16429, 1872),
+              (False, (256, 256), 388, 16429, 1872), (True, (32, 64), 259, 1030, 208), (True, (64, 128), 98, 12415, 208),
+              (True, (128, 128), 69, 16447, 1872), (True, (192, 128), 259, 13071, 1872)]
+
+
+@pytest.mark.parametrize("out_dt", ["half", "fp32"])
+@pytest.mark.parametrize("int8,tile,rows,n,k", TILE_CASES)
+def test_output_layouts_of_each_tile(pkg, cuda, int8, tile, rows, n, k, out_dt):
+    _check_layouts(cuda, rows, n, k, out_dt, int8)
+
+
 @pytest.mark.parametrize("int8", [False, True])
 @pytest.mark.parametrize("out_dt", ["half", "fp32"])
 @pytest.mark.parametrize("rows,n", [(130, 1032), (259, 1026), (300, 1029), (700, 3001), (1100, 9004)])
 def test_output_layouts(pkg, cuda, rows, n, out_dt, int8):
+    _check_layouts(cuda, rows, n, 208, out_dt, int8)
+
+
+def _check_layouts(cuda, rows, n, k, out_dt, int8):
     lib = importlib.import_module("llm-inference-optimizer_amd._lib").load()
     dt = F16 if n % 2 else BF16
-    k = 208
     g = torch.Generator(device="cuda").manual_seed(rows + n)
     x = torch.randn(rows, k, generator=gen(n)).to(dt).to(cuda)
     if int8:

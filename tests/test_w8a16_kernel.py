@@ -180,32 +180,25 @@ def test_decode_stream_kernel_matches_oracle(pkg, orc, cuda, M, K, N, dt, bias):
     assert torch.equal(got16, got32.to(dt)), "the 16-bit output must be the fp32 output rounded once"
 
 
-# Prefill shapes that land on each of the tiled GEMM's launch shapes (by the
-# number of 128 x 128 output tiles), with k tails and ragged edges.
+# Prefill shapes on the tiled GEMM, with k tails and ragged edges; the tile
+# that the plan takes on 256 CUs (each tile at ragged sizes: test_tiled_shapes.py).
 TILED_CASES = [
-    (300, 1552, 1000, F16, True),     # < 128 tiles: 64 x 64
-    (320, 512, 8960, F16, False),     # < 320: 128 x 128, 8 waves, step pipeline
-    (200, 2048, 8960, BF16, True),    # <= 256 rows but a large grid: tiled, 128 x 128
-    (4096, 256, 1536, F16, True),     # n <= 2048: 128 x 256
-    (4096, 256, 1536, BF16, False),   # (bf16: 128 x 128)
-    # n <= 2048 with between cus / 2 and cus tiles of 64 x 128: 8 waves, ring
-    (1024, 1536, 1536, F16, True),    # 192 tiles
-    (1000, 272, 2000, BF16, False),   # 256 tiles, ragged rows and n, k tail
-    # n > 2048 below 1024 rows with >= 2 tiles of 128 x 64 per CU: the sub-step ring
-    (512, 512, 8960, F16, False),     # 128 x 64, 4 waves (main loop and k tail)
-    # n > 2048 from 1024 rows, k <= 4096: 128 x 128 tiles of 8 waves, 3-stage ring
+    (300, 1552, 1000, F16, True),     # 32 x 64
+    (320, 512, 8960, F16, False),     # 64 x 64
+    (200, 2048, 8960, BF16, True),    # 128 x 128
+    (4096, 256, 1536, F16, True),     # 64 x 64
+    (4096, 256, 1536, BF16, False),
+    (1024, 1536, 1536, F16, True),    # 32 x 64
+    (1000, 272, 2000, BF16, False),   # 64 x 128, ragged rows and n, k tail
+    (512, 512, 8960, F16, False),     # 64 x 64
     (2048, 128, 8952, F16, False),    # ragged n
     (4096, 64, 8960, F16, True),
-    (4096, 80, 9000, BF16, True),     # ragged n, k tail only
-    (4096, 32, 3584, BF16, True),
-    # ... except where 192 x 128 tiles fit in one round of two workgroups per
-    # CU and 128 x 128 tiles do not: 192 x 128, registers capped at 128
-    (1024, 272, 8960, BF16, False),   # 420 tiles
-    (1200, 400, 8000, F16, True),     # 441 tiles: ragged rows and n, k tail
-    # n > 2048 with k > 4096 and many 128 x 64 tiles: the launch plan weighs
-    # rounds of 128 x 64, 256 x 128 and 256 x 256 tiles (sub-step ring)
-    (512, 4608, 14336, F16, True),    # 256 x 128, 8 waves of 128 x 32
-    (1024, 4608, 14336, BF16, False), # 256 x 256, 8 waves of 64 x 128
+    (4096, 80, 9000, BF16, True),     # ragged n, k tail
+    (4096, 32, 3584, BF16, True),     # k tail only
+    (1024, 272, 8960, BF16, False),
+    (1200, 400, 8000, F16, True),     # 192 x 128: ragged rows and n, k tail
+    (512, 4608, 14336, F16, True),    # 128 x 128
+    (1024, 4608, 14336, BF16, False),
     # 17 - 64 rows with >= 128 tile columns: the small tiled shapes
     (24, 1536, 8960, F16, True),      # 32 x 64
     (20, 256, 16400, BF16, False),    # n > 10000: 32 x 128
