@@ -22,10 +22,11 @@
 // at a full chip, longer than one step of most tiles, and the weights' copies
 // come from HBM, so where LDS cannot hold a third whole stage it holds one of
 // the weights: 256 x 128 gate/up tiles with S = 2, SB = 3 take 15 - 25% less
-// time per step at 1 - 2 rounds than with SB = 2.  Buffer descriptors end at the last valid element (rows
-// past the matrix read 0); the K step enters through the scalar offset, and
-// only a final partial step redirects columns at or past k past the
-// descriptor, so any k that is a multiple of 16 (int8) or 8 (16-bit) works.
+// time per step at 1 - 2 rounds than with SB = 2.  Buffer descriptors end at the
+// last valid element (rows past the matrix read 0); the K step enters through
+// the scalar offset, and only a final partial step redirects columns at or past
+// k past the descriptor, so any k that is a multiple of 16 (int8) or 8 (16-bit)
+// works.
 //
 // Two main loops.  The step pipeline (RING = 0, S >= 3): per step a wave
 // waits for its own DMA of the next step (vmcnt, the later steps stay in
@@ -68,8 +69,11 @@
 // visible to the compiler, whose waits for them drain the DMA pipeline.)
 //
 // Epilogue.  The MFMAs take b as their first operand, so each lane ends with
-// four consecutive output columns of one row per register group: 8-byte
-// stores (16 for fp32 out).
+// four consecutive output columns of one row per register group.  They cross
+// the wave through LDS so that an instruction stores whole 64-byte row
+// segments, 16 bytes a lane, where the output's rows are whole aligned 16-byte
+// packets; else each lane stores its own 8 bytes (16-bit rows of whole quads)
+// or single elements.
 //
 // Grid: one workgroup per tile, 1-D.  Consecutive workgroup ids land on
 // different XCDs (round robin over 8), so ids are remapped to give each XCD
@@ -153,12 +157,12 @@ struct Cfg {
   static constexpr int BI = B_BYTES / 1024 / NW;  // B DMA instructions per wave per step and matrix
   static constexpr int P = AI + NB * BI;          // DMA instructions per wave per step
   static_assert(A_BYTES % (1024 * NW) == 0 && B_BYTES % (1024 * NW) == 0, "tile must split over the waves");
-  // The operand with more stages is issued second in a step, so a wait for the
-  // next step leaves its younger copies, and WAIT instructions in all, in flight.
-  static constexpr int SMIN = S < SB ? S : SB, SMAX = S < SB ? SB : S;
-  static constexpr int WAIT = (SMIN - 2) * P + (S < SB ? NB * BI : (S > SB ? AI : 0));
+  // The weights, with as many stages or one more, are issued second in a step, so
+  // a wait for the next step leaves their younger copies, and WAIT instructions
+  // in all, in flight.
+  static constexpr int WAIT = (S - 2) * P + (S < SB ? NB * BI : 0);
   static constexpr int FILL = S * AI + SB * NB * BI;  // instructions that fill every stage
-  static_assert(SMIN >= 2 && SMAX <= 10, "2..10 stages");
+  static_assert(S >= 2 && (SB == S || SB == S + 1) && SB <= 10, "2..10 stages, the weights' as many or one more");
   static_assert(FILL - P < 64, "vmcnt range");
 };
 
@@ -604,7 +608,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
     };
     Sub rf;
     prefill(std::integral_constant<int, S>{}, std::integral_constant<int, SB>{});
-    if (C::SMAX - 1 < nk) wait_vmcnt<C::FILL - C::P>();
+    if (SB - 1 < nk) wait_vmcnt<C::FILL - C::P>();
     else wait_vmcnt<0>();
     wait_lgkmcnt0();
     lds_barrier();
@@ -621,17 +625,12 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
         if (s < 3) {
           read_one(std::integral_constant<int, sa>{}, std::integral_constant<int, sb>{}, rf, s + 1);
         } else if (more) {
-          if (!guard || t + C::SMAX - 1 < nk) wait_vmcnt<C::WAIT>();
+          if (!guard || t + SB - 1 < nk) wait_vmcnt<C::WAIT>();
           else wait_vmcnt<0>();
           wait_lgkmcnt0();
           lds_barrier();
-          if constexpr (S > SB) {
-            if (!guard || t + SB < nk) issue_b(std::integral_constant<int, sb>{}, t + SB);
-          }
           if (!guard || t + S < nk) issue_a(std::integral_constant<int, sa>{}, t + S);
-          if constexpr (S <= SB) {
-            if (!guard || t + SB < nk) issue_b(std::integral_constant<int, sb>{}, t + SB);
-          }
+          if (!guard || t + SB < nk) issue_b(std::integral_constant<int, sb>{}, t + SB);
           read_one(std::integral_constant<int, (sa + 1) % S>{}, std::integral_constant<int, (sb + 1) % SB>{}, rf, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -649,8 +648,8 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
       }
       __builtin_amdgcn_sched_barrier(0);
     };
-    // main loop: steps t0 .. t0 + UNROLL - 1 issue steps up to t0 + UNROLL + SMAX - 1 < kfull
-    for (; t0 + UNROLL + C::SMAX - 1 < kfull; t0 += UNROLL) {
+    // main loop: steps t0 .. t0 + UNROLL - 1 issue steps up to t0 + UNROLL + SB - 1 < kfull
+    for (; t0 + UNROLL + SB - 1 < kfull; t0 += UNROLL) {
       static_for([&](auto I) { rstep(I, std::false_type{}, t0 + decltype(I)::value); },
                  std::make_index_sequence<UNROLL>{});
     }
@@ -704,7 +703,7 @@ __attribute__((amdgpu_waves_per_eu(kMinWavesPerSimd<WPE>))) void tiled_gemm(cons
   for (int j = 0; j < FN; ++j) {
     const int nj = wn * FN * 32 + 32 * j;  // first column of the 32-column block in the tile
     // scale and bias (EPI_SILU_W8: up scale) of this lane's 16 columns, all
-    // loads in flight together; columns past the matrix repeat the last one
+    // loads in flight together; columns past the matrix read 0
     const int c0 = nj + 4 * eh;
     float sc[16], bz[16];
     if constexpr (EPI == EPI_W8 || EPI == EPI_SILU_W8) load_columns(sc, p.scale, p.sdt, ncol0, c0, ncols);

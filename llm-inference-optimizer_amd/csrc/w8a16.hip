@@ -430,8 +430,9 @@ int w8_typed(const W8Params& p, hipStream_t s, int cus, void* work = nullptr, in
   // One matrix of at least 17 rows whose output holds too few tiles for the
   // CUs: split K (split_k.h has the figures), where the plan predicts it
   // faster than the kernels below.
+  tiled::SplitPlan sp{};
   if constexpr (!DUAL) {
-    const tiled::SplitPlan sp = tiled::split_plan(p.rows, p.k, p.n, 1, cus);
+    sp = tiled::split_plan(p.rows, p.k, p.n, 1, cus);
     if (sp.tile >= 0 && work != nullptr && work_bytes >= tiled::split_bytes(sp, p.rows, p.n) && tiled_fits(p, DUAL))
       return tiled::split_k_launch<T, tiled::B_I8, TO, tiled::EPI_W8>(w8_tiled_params(p, p.q), sp,
                                                                        static_cast<float*>(work), s);
@@ -472,7 +473,7 @@ int w8_typed(const W8Params& p, hipStream_t s, int cus, void* work = nullptr, in
   const bool skinny = tiled::w8_skinny_pays(p.rows, p.n) || !tiled_fits(p, DUAL);
   if (skinny) return w8_skinny_shape<T, TO, 4, DUAL>(p, s, cus);
   if constexpr (DUAL) return w8_tiled_dual<T, TO>(p, s, cus);
-  else return w8_tiled<T, TO>(p, tiled::split_plan(p.rows, p.k, p.n, 1, cus).direct, s);
+  else return w8_tiled<T, TO>(p, sp.direct, s);
 }
 
 }  // namespace
