@@ -74,7 +74,7 @@ def parse_args():
                                       "gate-up-prefill", "gate-up-w8", "gate-up-w8-decode", "w8a16", "w8a16-decode", "decode-wide-rows",
                                       "w8a16-prefill", "w8a16-prefill-1.5b", "prefill-core",
                                       "gate-up-w8-prefill", "w8a16-prefill-wide", "w8a16-prefill-narrow",
-                                      "gate-up-prefill-sweep", "w8a16-prefill-ragged", "w8-decomp", "w8-layouts", "w8-layouts8", "w8-stream-sweep", "gu16-stream-sweep", "stream-sweep16", "stream-sweep16-wide", "stream-sweep-r8", "stream-sweep-m4", "stream-sweep16-k", "stream-sweep-dualn", "stream-sweep-dual32", "stream-sweep-3b14b", "stream-sweep-bal", "stream-sweep-few16", "stream-sweep-dual4", "stream-sweep-14b-wide", "stream-sweep-smallm", "l16-stream-sweep", "stream-sweep32", "stream-sweep64", "stage3",
+                                      "gate-up-prefill-sweep", "tile-plans", "w8a16-prefill-ragged", "w8-decomp", "w8-layouts", "w8-layouts8", "w8-stream-sweep", "gu16-stream-sweep", "stream-sweep16", "stream-sweep16-wide", "stream-sweep-r8", "stream-sweep-m4", "stream-sweep16-k", "stream-sweep-dualn", "stream-sweep-dual32", "stream-sweep-3b14b", "stream-sweep-bal", "stream-sweep-few16", "stream-sweep-dual4", "stream-sweep-14b-wide", "stream-sweep-smallm", "l16-stream-sweep", "stream-sweep32", "stream-sweep64", "stage3",
                                       "e2e-compact", "e2e-int8-compact"],
                    default=None,
                    help="run one kernel loop only (for profiler runs)")
@@ -1075,6 +1075,10 @@ def run_only(ctx, args, sets):
         del sets
         torch.cuda.empty_cache()
         print(json.dumps({"gate_up16_stream_sweep": gu16_stream_sweep(ctx)}), flush=True)
+    elif args.only == "tile-plans":  # the plans' predicted times against measured ones
+        del sets
+        torch.cuda.empty_cache()
+        print(tile_plan_table(ctx), flush=True)
     elif args.only == "stream-sweep32":  # 17 - 32 rows: all three forms of the decode kernel
         del sets
         torch.cuda.empty_cache()
@@ -2207,6 +2211,78 @@ def bench_linear16(ctx, shapes=LINEAR16_SHAPES, iters=300, baselines=True):
         del ws, outs, calls
         torch.cuda.empty_cache()
     return res
+
+
+# (hidden, intermediate) of the Qwen2.5 sizes the tile plans were fitted on, and prompt-sized row counts
+TILE_PLAN_DIMS = ((896, 4864), (1536, 8960), (2048, 11008), (3584, 18944), (5120, 13824))
+TILE_PLAN_ROWS = (72, 100, 160, 256, 333, 512, 700, 1000, 1536, 2048, 3000, 4096)
+
+
+def tile_plan_table(ctx, dims=TILE_PLAN_DIMS, rows=TILE_PLAN_ROWS):
+    """The time that the tile and split-K plans predict for the launch they
+    choose against that launch measured (hipGraph, weights rotated through
+    HBM, fp16), over the Qwen2.5 projections at more than 64 rows: a markdown
+    table per kernel, with the mean error and bias.  (Calls that leave the
+    tiled kernels are not listed.)"""
+    torch = ctx.torch
+    F16, ll, i32 = torch.float16, ctypes.c_longlong, ctypes.c_int
+    tile = ctx.probe.mi355_probe_tile_plan
+    tile.argtypes, tile.restype = [i32, ll, ll, ll, i32, ctypes.POINTER(i32)], ctypes.c_double
+    split = ctx.probe.mi355_probe_split_plan
+    split.argtypes, split.restype = [ll, ll, ll, i32, i32, ctypes.POINTER(i32)], ll
+    cost = ctx.probe.mi355_probe_split_cost
+    cost.argtypes, cost.restype = [ll, ll, ll, i32, i32, ctypes.POINTER(ctypes.c_double)], None
+    cus = torch.cuda.get_device_properties(ctx.dev).multi_processor_count
+    t9, s4, c2 = (i32 * 9)(), (i32 * 4)(), (ctypes.c_double * 2)()
+    g = torch.Generator(device=ctx.dev)
+    g.manual_seed(7)
+    out = []
+    for table, name, wb, mats in ((0, "16-bit linear", 2, 1), (1, "int8 linear", 1, 1), (2, "16-bit gate/up", 2, 2),
+                                  (3, "int8 gate/up", 1, 2)):
+        lines, err = [], {"unsplit": [], "split K": []}
+        shapes = [(h, i) for h, i in dims]
+        if mats == 1:
+            shapes = [s for h, i in dims for s in ((h, h), (i, h), (h, i))]
+        for k, n in shapes:
+            sets = min(40, max(2, n_sets(mats * n * k * wb)))
+            if wb == 1:
+                ws = [(torch.randint(-127, 128, (mats, n, k), generator=g, device=ctx.dev, dtype=torch.int8),
+                       torch.rand(mats, n, generator=g, device=ctx.dev) * 1e-3) for _ in range(sets)]
+            else:
+                ws = [(rand(ctx, (mats, n, k), 40 + i, F16, std=k ** -0.5), None) for i in range(sets)]
+            for m in rows:
+                x, o = rand(ctx, (m, k), m, F16), torch.empty((m, n), dtype=F16, device=ctx.dev)
+                tiles64 = -(-n // 64) * -(-m // 64)
+                if wb == 1 and m <= 256 and (tiles64 < 32 or (m <= 128 and n < 2048)):
+                    continue  # 32-row tiles of the W8A16 kernels' own
+                us, kind = tile(table, m, k, n, cus, t9), "unsplit"
+                plan = f"{t9[3]} x {t9[4]}"
+                if t9[1]:
+                    plan += f" over {t9[1]} columns, then {t9[6]} x {t9[7]}"
+                if mats == 1 and split(m, k, n, wb, cus, s4) > 0:
+                    cost(m, k, n, wb, cus, c2)
+                    us, kind, plan = c2[0], "split K", f"{s4[2]} x {s4[3]}, {s4[1]} ranges"
+                if mats == 2:
+                    calls = [ctx.gate_up_w8_call(x, w[0], s[0], w[1], s[1], o) if wb == 1 else
+                             ctx.gate_up_call(x, w[0], w[1], o) for w, s in ws]
+                else:
+                    calls = [ctx.w8a16_call(x, w[0], s[0], o) if wb == 1 else ctx.linear16_call(x, w[0], o)
+                             for w, s in ws]
+                spin_up(ctx, calls, ms=4.0)
+                got = time_graph(ctx, calls, max(sets, 20), replays=3)
+                err[kind].append(us / got - 1)
+                lines.append(f"| {m} | {k} | {n} | {plan} | {us:.1f} | {got:.1f} | {us / got - 1:+.0%} |")
+            del ws
+            torch.cuda.empty_cache()
+        out.append(f"## {name}\n")
+        for kind, e in err.items():
+            if e:
+                out.append(f"{kind}: {len(e)} sizes, mean error {statistics.mean(map(abs, e)):.1%}, bias "
+                           f"{statistics.mean(e):+.1%}, from {min(e):+.0%} to {max(e):+.0%}.")
+        out += ["", "| rows | k | n | launch | predicted us | measured us | error |", "|---|---|---|---|---|---|---|",
+                *lines, ""]
+        log(f"  tile plans, {name}: {len(lines)} sizes")
+    return "\n".join(out)
 
 
 def w8a16_kernel_name(M, N, K=0, workspace=0):

@@ -141,7 +141,8 @@ int l16_tiled_cfg(const L16Params& p, hipStream_t s) {
 // and 3).  (The rule before -- 64 x 64 below 128 tiles of 128 x 128, else
 // those in the step pipeline -- took 3B q/o at 1000 rows 16.9 us, now 12.9;
 // the 14B q/o at 333 rows 45.1, now 36.8; over the Qwen2.5-0.5B to 14B
-// projections at 72 - 4096 rows the plan takes 0.87 of its time.)
+// projections at 72 - 4096 rows the plan takes 0.87 of its time.)  256 x 256
+// fills the register file: 24 bytes a lane live in scratch.
 template <typename T, typename TO>
 int l16_tiled(const L16Params& p, int shape, hipStream_t s) {
   switch (shape) {

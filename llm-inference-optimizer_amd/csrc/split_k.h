@@ -10,16 +10,16 @@
 // of 76 - 296 K steps.  S = CUs / tiles ranges give every CU a workgroup and
 // cut the chain by S, for 8 S rows n bytes of extra traffic (fp32 sums
 // written once and read once, L2 and Infinity Cache hits) and a second
-// launch.  Measured on MI355X, weights from HBM, before (the stream kernel up
-// to 64 rows, unsplit tiles beyond) and after, both passes:
-//   7B down (18944 -> 3584), 16-bit:  64 rows 80.6 -> 32.0 us, 200 rows 79.3
-//     -> 52.3, 512 rows 153 -> 85.4, 1000 rows 168 -> 134 (1.01 PFLOP/s);
-//     int8: 64 rows 82.3 -> 25.8, 200 rows 82.2 -> 46.3, 512 rows 123 -> 88
-//   1.5B down (8960 -> 1536), 16-bit: 64 rows 19.9 -> 13.3, 200 rows 38.1 ->
-//     18.8, 1000 rows 70.8 -> 46.8; int8: 64 rows 29.1 -> 12.4, 200 rows 38.9
-//     -> 18.3, 1000 rows 49.2 -> 41.9
-// What bounds it: HBM on the weights up to about 64 rows (16-bit: 4.8 TB/s
-// in the first pass alone), per-step latency of one workgroup per CU above;
+// launch.  Measured on MI355X, fp16, weights from HBM, unsplit (the stream
+// kernel or skinny tiles up to 64 rows, the tiles of tiled_plan.h beyond) and
+// split, both passes:
+//   7B down (18944 -> 3584), 16-bit:  64 rows 79.1 -> 36.9 us, 200 rows 78.4
+//     -> 52.6, 512 rows 119 -> 85.5, 1000 rows 167 -> 144;
+//     int8: 64 rows 80.5 -> 27.0, 200 rows 76.8 -> 46.0, 512 rows 107 -> 89
+//   1.5B down (8960 -> 1536), 16-bit: 64 rows 22.5 -> 13.1, 200 rows 36.1 ->
+//     19.4, 512 rows 39.4 -> 29.2; int8: 64 rows 28.7 -> 13.0, 200 rows 34.8
+//     -> 19.3, 1000 rows 48.6 -> 43.3
+// What bounds it: HBM on the weights up to about 64 rows, per-step latency of one workgroup per CU above;
 // the second pass costs about 3 us and its launch about 3 more in a stream.
 //
 // Every output's sum is taken in one fixed order (range by range, each in
@@ -88,8 +88,9 @@ __global__ __launch_bounds__(256) void split_k_reduce(const Params p) {
 // one after another) + part * (MB of fp32 sums written and read) + weight *
 // (MB of weights).  Least-squares fits of a sweep on MI355X over the
 // Qwen2.5-0.5B to 14B down projections and square projections (896 - 5120
-// outputs, k 1536 - 18944) at 24 - 1500 rows, weights rotated through HBM:
-// mean error 2 - 5% per tile.
+// outputs, k 1536 - 18944) at 24 - 1500 rows, weights rotated through HBM: on
+// the kernels as they are, mean error 5% (int8 3% high) over the launches it
+// chooses at 72 - 4096 rows.
 struct TileCost {
   int bm, bn;
   double c0, step, part, weight;

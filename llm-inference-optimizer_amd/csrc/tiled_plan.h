@@ -20,7 +20,10 @@ namespace tiled {
 // chip lowers its clock: 1.8 GHz under these kernels at long prompts).  The
 // constants are least-squares fits (non-negative) to sweeps on MI355X over the
 // Qwen2.5-0.5B to 14B projections at 33 - 4096 rows, weights rotated through
-// HBM; mean error 3 - 7% per shape.
+// HBM, made before the epilogue stored whole row segments and loaded its scales
+// together.  Against the kernels as they are the chosen launches' mean error is
+// 7% for the 16-bit linear and both gate/ups and 13% for the int8 linear, which
+// is predicted 12% high throughout (bench.py --only tile-plans).
 // `round` is a tile's first loads and its epilogue, which nothing overlaps
 // where a CU holds one workgroup.
 struct ShapeCost {

@@ -9,10 +9,10 @@ a handful of rows and hipBLASLt runs it well below HBM bandwidth.  Here up to
 32 rows (64 on narrow outputs) read every weight byte once, at HBM
 bandwidth, on MFMA; more rows run an LDS-tiled MFMA GEMM, split over K (from
 17 rows) where the output alone would not fill the chip.  Sums are fp32 in
-this library's own order and the bias is added in fp32 before the one rounding to x's dtype, so results may
-differ from torch's linear in the last output bit.  FusedMLP uses it only on
-request (``hip_down=True``) and only for inputs of at most ``LINEAR16_MAX_ROWS``
-rows, where it is faster than hipBLASLt.
+this library's own order and the bias is added in fp32 before the one rounding
+to x's dtype, so results may differ from torch's linear in the last output bit.
+FusedMLP uses it only on request (``hip_down=True``) and only for inputs of at
+most ``LINEAR16_MAX_ROWS`` rows.
 """
 from __future__ import annotations
 
@@ -22,8 +22,10 @@ from .. import _lib
 
 __all__ = ["linear16", "LINEAR16_MAX_ROWS"]
 
-# Rows up to which FusedMLP's down projection takes this kernel (one 32-row
-# weight-streaming tile); larger inputs stay on torch's linear.
+# Rows up to which FusedMLP's down projection takes this kernel; larger inputs
+# stay on torch's linear.  The line was drawn where the weight-streaming kernel
+# and the unsplit tiles stopped being faster than hipBLASLt; split K has since
+# made 33 rows and more faster, and the comparison was not repeated.
 LINEAR16_MAX_ROWS = 32
 
 
