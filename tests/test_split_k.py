@@ -5,6 +5,7 @@ the GPU -- within one output ulp plus the worst-case fp32 summation error,
 the fp32 output within that bound, the 16-bit output equal to the fp32 output
 rounded once -- and against the unsplit kernels the C ABI runs without a
 workspace.  Also under graph replay and with row-strided inputs."""
+import gc
 import importlib
 
 import pytest
@@ -138,9 +139,7 @@ def test_without_memory_for_the_workspace(pkg, cuda, lib, int8):
     """A call whose output fits but whose workspace does not runs the unsplit
     kernels, as one through the C ABI without a workspace does."""
     rows, k, n = 700, 18944, 3584
-    torch.cuda.empty_cache()
     x, w, s, call = _linear(pkg, cuda, int8, rows, k, n)
-    torch.cuda.empty_cache()  # every tensor of the test in a segment of its own
     want = torch.empty(rows, n, dtype=F16, device=cuda)
     stream = torch.cuda.current_stream().cuda_stream
     if int8:
@@ -151,16 +150,22 @@ def test_without_memory_for_the_workspace(pkg, cuda, lib, int8):
         nbytes = lib.load().mi355_linear16_workspace(rows, k, n)
         lib.linear16_fwd(x.data_ptr(), w.data_ptr(), None, want.data_ptr(), rows, k, n, k, k, n, lib.F16, 0, lib.F16,
                          stream)
-    assert nbytes > 20 << 20, "must not fit the segment of the cached block below"
+    assert nbytes > 20 << 20, "more than a segment that the allocator makes for the output"
     torch.cuda.synchronize()
-    torch.cuda.empty_cache()
-    torch.empty(rows, n, dtype=F16, device=cuda)  # freed: a cached block for the output
+    room, fill = torch.empty_like(want), []
+    gc.collect()
     try:
         torch.cuda.set_per_process_memory_fraction(
             torch.cuda.memory_reserved() / torch.cuda.get_device_properties(cuda).total_memory)
+        # what other tests left free, down to gaps and a remainder that hold no output
+        for size in (nbytes, want.numel() * 2):
+            with pytest.raises(torch.OutOfMemoryError):
+                while True:
+                    fill.append(torch.empty(size, dtype=torch.uint8, device=cuda))
+        del room  # the one block for the output, between blocks in use
+        got = call()
         with pytest.raises(torch.OutOfMemoryError):
             torch.empty(nbytes, dtype=torch.uint8, device=cuda)
-        got = call()
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert torch.equal(got, want)
