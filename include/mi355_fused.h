@@ -191,7 +191,7 @@ int mi355_w8a16_linear_fwd(const void* x, const void* w_q, const void* scale, co
 
 /*
  * The same with a workspace, which lets calls of 17 to about 1500 rows whose
- * output is narrow split K over the GPU (two kernels, no allocation).
+ * output holds too few tiles for the CUs split K (two kernels, no allocation).
  * mi355_w8a16_linear_workspace returns the bytes such a call wants on the
  * current device, 0 where it would not use them; `workspace` is 16-byte
  * aligned device memory of `workspace_bytes` that no other work touches until
