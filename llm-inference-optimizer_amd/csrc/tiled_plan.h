@@ -29,6 +29,7 @@ namespace tiled {
 struct ShapeCost {
   int bm, bn, threads, occ;  // threads per workgroup
   double c0, step[3], load, weight, round;
+  double least;  // a K step of a last round takes no less, however few its tiles
 };
 
 // (32-bit divisions: the plan runs in every call; with 64-bit ones it cost a
@@ -49,7 +50,14 @@ __attribute__((always_inline)) inline double shape_time(const ShapeCost& s, uint
   const uint32_t slots = cus * static_cast<uint32_t>(s.occ);
   const uint32_t full = tiles / slots, rest = tiles - full * slots;
   double per_step = full * s.step[s.occ - 1] + s.load * tiles / cus;
-  if (rest > 0) per_step += s.step[(rest > cus) + (rest > 2 * cus)];
+  if (rest > 0) {
+    const double last = s.step[(rest > cus) + (rest > 2 * cus)];
+    per_step += last;
+    if (s.least > 0) {
+      const double with_load = last + s.load * rest / cus;
+      if (with_load < s.least) per_step += s.least - with_load;
+    }
+  }
   return s.c0 + s.round * (full + (rest > 0)) + plan_cdiv(k, 64u) * per_step + s.weight * wmb;
 }
 
@@ -116,14 +124,17 @@ constexpr ShapeCost kW8Cost[] = {{64, 64, 256, 3, 6.1, {0.181, 0.262, 0.400}, 0.
                                  {192, 128, 512, 2, 3.0, {0.429, 0.761, 0}, 0.322, 0, 6.5},
                                  {32, 64, 128, 3, 5.5, {0.177, 0.262, 0.282}, 0.022, 0.052, 0}};
 // One 16-bit matrix (linear16.hip): 64 x 64, 128 x 64, 64 x 128, 128 x 128 (one
-// and two per CU), 256 x 128 and 256 x 256.
+// and two per CU), 256 x 128 and 256 x 256.  (A step of one 256 x 256 tile is
+// 0.86 us of MFMA at the peak rate; the fit had no round of few such tiles and
+// priced one of 24 at 0.51 us: 14B down, 3500 rows, 280 tiles, 496 us predicted,
+// 613 measured, where 256 x 128 tiles take 534.)
 constexpr ShapeCost kL16Cost[] = {{64, 64, 256, 2, 2.0, {0.213, 0.368, 0}, 0, 0.138, 0.8},
                                   {128, 64, 256, 2, 3.2, {0.259, 0.533, 0}, 0.017, 0.126, 1.8},
                                   {64, 128, 512, 1, 1.2, {0.235, 0, 0}, 0.048, 0.164, 2.2},
                                   {128, 128, 512, 1, 1.5, {0.298, 0, 0}, 0.170, 0.126, 3.0},
                                   {128, 128, 512, 2, 2.4, {0.363, 0.433, 0}, 0.263, 0.085, 2.7},
                                   {256, 128, 512, 1, 0, {0.523, 0, 0}, 0.277, 0.011, 9.6},
-                                  {256, 256, 512, 1, 0, {0.397, 0, 0}, 1.198, 0, 20.9}};
+                                  {256, 256, 512, 1, 0, {0.397, 0, 0}, 1.198, 0, 20.9, 1.05}};
 // 16-bit gate/up + SiLU-and-mul (gate_up_silu.hip): 64 x 64, 128 x 64, 128 x
 // 128, 192 x 128, 256 x 128 and 256 x 64.
 constexpr ShapeCost kGateUpCost[] = {{64, 64, 256, 2, 1.7, {0.328, 0.551, 0}, 0.055, 0.101, 0},

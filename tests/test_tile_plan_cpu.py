@@ -100,3 +100,13 @@ def test_store_cases_take_the_tiles_they_name():
         assert tile_plan(table, rows, k, n)[4][:2] == tile, (rows, k, n)
     assert {t for int8, t, *_ in stores.TILE_CASES if int8} == {(32, 64), (64, 128), (128, 128), (192, 128)}
     assert {t for int8, t, *_ in stores.TILE_CASES if not int8} == {(128, 64), (64, 128), (128, 128), (256, 128), (256, 256)}
+
+
+@pytest.mark.parametrize("rows,k,n", [(3500, 13824, 5120), (3400, 13824, 5120), (4352, 18944, 4096)])
+def test_linear16_takes_no_thin_round_of_its_largest_tile(rows, k, n):
+    """256 x 256 tiles that leave a last round of a few (280, 280 and 272 on 256
+    CUs) cost a whole tile's chain: smaller ones measured faster."""
+    if not PROBE.exists():
+        pytest.skip("probe library not built")
+    assert 256 < -(-rows // 256) * -(-n // 256) < 300
+    assert tile_plan(LINEAR16, rows, k, n)[4][:2] != (256, 256)
